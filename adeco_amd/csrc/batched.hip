@@ -51,6 +51,7 @@
 #include "kernels.hpp"
 #include "octree_impl.hpp"
 #include "runtime.hpp"
+#include "wave_tiles.hpp"
 
 namespace adeco {
 
@@ -71,6 +72,12 @@ GridDesc make_grid_desc(const GridGeom& g, long long base) {
     return d;
 }
 
+int deposit_form(int precision, const GridDesc* grids, int64_t n) {
+    bool unit = precision == ADECO_PREC_FP64;
+    for (int64_t i = 0; i < n && unit; ++i) unit = grids[i].r[0] == 1.0 && grids[i].r[1] == 1.0 && grids[i].r[2] == 1.0;
+    return unit ? int(kFormBlocks) : precision;
+}
+
 LaunchShape& launch_shape() {
     static LaunchShape s;
     return s;
@@ -82,8 +89,6 @@ constexpr int kWavesPerBlock = 4;
 constexpr int kBlock = 64 * kWavesPerBlock;
 constexpr int kBuckets = 23;       // 22 clip work classes + the exact-recompute queue
 constexpr int kExactQueue = 22;
-// launches with fewer tiles than this per resident wave drain their queues in merged passes
-constexpr int64_t kMergeDrainTiles = 16;
 // how a wave drains its queues once the work items run out: a pass per queue (a large launch or a
 // step of the request server), or passes filled from all the classes (a small launch)
 constexpr int kDrainPerClass = 0, kDrainAll = 1;
@@ -109,16 +114,6 @@ struct WaveLds {
     float sab[kMaxSeg][kWaveTile];    // sums of their magnitudes (the noise threshold's scale)
 };
 static_assert(kBuckets <= 24 && kBuckets < 32, "queue counts and the drain's prefix sum cover 24 lanes");
-
-__device__ __forceinline__ int upper_bound_i64(const int64_t* a, int n, int64_t v) {
-    int lo = 0, hi = n;
-    while (lo < hi) {
-        const int mid = (lo + hi) >> 1;
-        if (a[mid] <= v) lo = mid + 1;
-        else hi = mid;
-    }
-    return lo;
-}
 
 // per pair: PairData and candidate count (dead pairs keep one dummy candidate so every pair owns
 // at least one candidate and a tile of 64 candidates spans at most 64 pairs).  With columns
@@ -474,59 +469,6 @@ __device__ __forceinline__ int work_class(const V3<double> s[4], const double mn
     return 18 + (t1 <= 1 ? 0 : 1 + t2);                                       // 18-21
 }
 
-// n / d for n < 2^30 and 1 <= d < 2^30 without the integer division sequence: the FP64 reciprocal
-// refined once is accurate to ~2^-50, so the truncated product is the quotient or one less (exact
-// multiples), fixed by one integer correction each way
-__device__ __forceinline__ unsigned udiv_small(unsigned n, unsigned d) {
-    const double dd = double(d);
-    double r = __builtin_amdgcn_rcp(dd);
-    r = fma(fma(-dd, r, 1.0), r, r);
-    unsigned q = unsigned(double(n) * r);
-    q -= unsigned(q * d > n);
-    q += unsigned((q + 1) * d <= n);
-    return q;
-}
-
-__device__ __forceinline__ void wave_sync() {
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
-
-__device__ __forceinline__ int64_t shfl_i64(int64_t v, int src) {
-    const int lo = __shfl(int(uint64_t(v) & 0xffffffffu), src, 64);
-    const int hi = __shfl(int(uint64_t(v) >> 32), src, 64);
-    return int64_t((uint64_t(unsigned(hi)) << 32) | unsigned(lo));
-}
-
-// What a tile's classification needs first: its source slot and index, its first pair, the number
-// of pairs it touches and, per lane, the candidate offset of pair p0 + lane.  Loaded one tile
-// ahead, so that these dependent loads overlap the previous tile's work.
-struct TileHead {
-    int slot;
-    int p0, np;
-    int64_t t;
-    int64_t my_off;
-};
-
-template <class Sources>
-__device__ __forceinline__ TileHead load_head(const Sources& srcs, const int2* __restrict__ entries, int64_t item,
-                                              int lane) {
-    TileHead h;
-    h.slot = 0;
-    h.t = item;
-    if (entries) {
-        const int2 en = entries[item];
-        h.slot = __builtin_amdgcn_readfirstlane(en.x);
-        h.t = int64_t(__builtin_amdgcn_readfirstlane(en.y));
-    }
-    const TileSource& src = srcs.get(h.slot);
-    h.p0 = src.tile_first[h.t];
-    h.np = min(src.tile_first[h.t + 1] - h.p0 + 1, kWaveTile);
-    h.my_off = lane < h.np ? src.cand_off[h.p0 + lane] : int64_t(0);
-    return h;
-}
-
 // Classifies the 64 candidates of tile h.t of `src` (slot h.slot among the launch's sources):
 // segments inside the tet and tets inside a single cell are deposited, partial candidates are
 // appended to the wave's queues.
@@ -714,15 +656,6 @@ __device__ __forceinline__ unsigned clip_entry(const Sources& srcs, int2 e, int 
     return redo;
 }
 
-struct OneSource {
-    TileSource s;
-    __device__ const TileSource& get(int) const { return s; }
-};
-struct ManySources {
-    const TileSource* s;
-    __device__ const TileSource& get(int i) const { return s[i]; }
-};
-
 // The persistent loop of one wavefront over work items [0, n_items): item -> (source slot, tile)
 // directly (one source) or through `entries`.  The wave pops `chunk` items per work-queue access;
 // a queue reaching 64 entries is clipped at once; when the items run out the queues are drained.
@@ -888,18 +821,10 @@ __global__ void k_zero_words(unsigned* p, int n) {
 
 inline size_t align256(size_t b) { return (b + 255) & ~size_t(255); }
 
-// Resident workgroups of a launch: blocks_per_cu per CU, capped at what the kernel's registers
-// and LDS let a CU hold (a surplus workgroup would only start once a resident one had drained the
-// work queue).
-int resident_blocks(int device, int precision, bool merge) {
-    int cus = 256;
-    (void)hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, device);
-    return cus * std::max(1, std::min(launch_shape().blocks_per_cu, deposit_occupancy(precision, merge)));
-}
-
 }  // namespace
 
 int deposit_occupancy(int precision, bool merge) {
+    if (precision == kFormBlocks) return block_occupancy();
     // per (precision, merge) instantiation of k_deposit_waves; k_deposit_step shares its resources
     static std::atomic<int> cache[3][2];
     const int pi = precision == ADECO_PREC_FP64 ? 0 : (precision == ADECO_PREC_MIXED ? 1 : 2);
@@ -947,7 +872,7 @@ hipError_t launch_scan_u32(const unsigned* in, int64_t n, int64_t* out, int64_t*
 // candidate scan; n_dev (nullable) is the pair count on the device, capped at n_pairs.
 static void enqueue_candidate_space(hipStream_t stream, const LatticeView& lat, const PackedCorners& ct,
                                     const int32_t* pairs, int64_t n_pairs, const int64_t* n_dev, const int64_t* grid_off,
-                                    int n_grids, const GridDesc* d_grids, double tet_mass, int precision, void* slab,
+                                    int n_grids, const GridDesc* d_grids, double tet_mass, int form, void* slab,
                                     CandidateSpace& cs) {
     char* w = static_cast<char*>(slab);
     const int64_t nblk = (n_pairs + kScanBlock - 1) / kScanBlock;
@@ -963,14 +888,19 @@ static void enqueue_candidate_space(hipStream_t stream, const LatticeView& lat, 
     w += align256(8);
     int32_t* pair_grid = n_grids > 1 ? reinterpret_cast<int32_t*>(w) : nullptr;
     cs.n_pairs = n_pairs;
+    cs.form = form;
     cs.n_cand = 0;
     cs.n_tiles = 0;
     if (n_pairs == 0) return;
     if (pair_grid)
         hipLaunchKernelGGL(k_pair_grid, dim3(unsigned(n_grids)), dim3(256), 0, stream, grid_off, n_pairs, pair_grid);
-    hipLaunchKernelGGL(k_pair_setup, dim3(unsigned((n_pairs + 255) / 256)), dim3(256), 0, stream, lat, ct, pairs, n_pairs,
-                       n_dev, grid_off, n_grids, pair_grid, d_grids, tet_mass, precision == ADECO_PREC_FP64 ? kMaxSeg : 1,
-                       cs.cand, cs.pd);
+    if (form == kFormBlocks)
+        (void)launch_block_setup(stream, lat, ct, pairs, n_pairs, n_dev, grid_off, n_grids, pair_grid, d_grids, tet_mass,
+                                 cs.cand, cs.pd);
+    else
+        hipLaunchKernelGGL(k_pair_setup, dim3(unsigned((n_pairs + 255) / 256)), dim3(256), 0, stream, lat, ct, pairs, n_pairs,
+                           n_dev, grid_off, n_grids, pair_grid, d_grids, tet_mass, form == kFormFp64 ? kMaxSeg : 1, cs.cand,
+                           cs.pd);
     hipLaunchKernelGGL(k_scan_reduce, dim3(unsigned(nblk)), dim3(256), 0, stream, cs.cand, n_pairs, n_dev, cs.block_sum);
     hipLaunchKernelGGL(k_scan_sums, dim3(1), dim3(kScanSumsBlock), 0, stream, cs.block_sum, nblk, cs.total);
     hipLaunchKernelGGL(k_scan_apply, dim3(unsigned(n_pairs / kScanBlock + 1)), dim3(256), 0, stream, cs.cand, n_pairs,
@@ -979,10 +909,9 @@ static void enqueue_candidate_space(hipStream_t stream, const LatticeView& lat, 
 
 adeco_status build_candidate_space(hipStream_t stream, const LatticeView& lat, const PackedCorners& ct,
                                    const int32_t* pairs, int64_t n_pairs, const int64_t* grid_off, int n_grids,
-                                   const GridDesc* d_grids, double tet_mass, int precision, void* slab,
+                                   const GridDesc* d_grids, double tet_mass, int form, void* slab,
                                    CandidateSpace& cs) {
-    enqueue_candidate_space(stream, lat, ct, pairs, n_pairs, nullptr, grid_off, n_grids, d_grids, tet_mass, precision,
-                            slab, cs);
+    enqueue_candidate_space(stream, lat, ct, pairs, n_pairs, nullptr, grid_off, n_grids, d_grids, tet_mass, form, slab, cs);
     if (n_pairs == 0) return ADECO_OK;
     hipError_t e = hipGetLastError();
     if (e == hipSuccess) e = hipMemcpyAsync(&cs.n_cand, cs.total, 8, hipMemcpyDeviceToHost, stream);
@@ -1004,10 +933,9 @@ adeco_status build_tile_map(hipStream_t stream, CandidateSpace& cs, int32_t* til
 hipError_t enqueue_candidate_space_dev(hipStream_t stream, const LatticeView& lat, const PackedCorners& ct,
                                        const int32_t* pairs, int64_t pair_cap, const int64_t* n_dev,
                                        const int64_t* grid_off, int n_grids, const GridDesc* d_grids, double tet_mass,
-                                       int precision, void* slab, int32_t* tiles, int64_t tile_cap, int64_t* sizes,
+                                       int form, void* slab, int32_t* tiles, int64_t tile_cap, int64_t* sizes,
                                        unsigned* overflow, CandidateSpace& cs) {
-    enqueue_candidate_space(stream, lat, ct, pairs, pair_cap, n_dev, grid_off, n_grids, d_grids, tet_mass, precision, slab,
-                            cs);
+    enqueue_candidate_space(stream, lat, ct, pairs, pair_cap, n_dev, grid_off, n_grids, d_grids, tet_mass, form, slab, cs);
     hipLaunchKernelGGL(k_space_sizes, dim3(1), dim3(1), 0, stream, cs.cand_off, n_dev, pair_cap, tile_cap, sizes, overflow);
     cs.tile_first = tiles;
     hipLaunchKernelGGL(k_tile_map, dim3(unsigned((pair_cap + 1 + 255) / 256)), dim3(256), 0, stream, cs.cand_off, pair_cap,
@@ -1015,71 +943,54 @@ hipError_t enqueue_candidate_space_dev(hipStream_t stream, const LatticeView& la
     return hipGetLastError();
 }
 
-hipError_t launch_deposit_tiles(hipStream_t stream, int precision, const TileSource& src, unsigned* queue_counter,
+WaveLaunch wave_launch(int64_t n_items, int occupancy, int waves, int device) {
+    int cus = 256;
+    (void)hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, device);
+    // resident workgroups: blocks_per_cu per CU, capped at what a CU holds (a surplus workgroup would only
+    // start once a resident one had drained the work queue)
+    const int64_t resident = int64_t(cus) * std::max(1, std::min(launch_shape().blocks_per_cu, occupancy));
+    WaveLaunch w;
+    w.chunk = int(std::max<int64_t>(1, std::min<int64_t>(launch_shape().chunk, n_items / (resident * waves))));
+    w.merge = n_items < kMergeDrainTiles * resident * waves;
+    const int64_t needed = (n_items + w.chunk - 1) / w.chunk;
+    w.grid = unsigned(std::max<int64_t>(1, std::min<int64_t>((needed + waves - 1) / waves, resident)));
+    return w;
+}
+
+hipError_t launch_deposit_tiles(hipStream_t stream, const TileSource& src, unsigned* queue_counter,
                                 unsigned long long* counters, int device) {
     if (src.n_tiles <= 0) return hipSuccess;
-    // small launches: fewer tiles per pop when there are too few to give every resident wave
-    // `chunk` of them, and drain passes that merge the work classes
-    // (the merged-drain instantiation decides with the large one's occupancy; it is the same or
-    // lower, and resident_blocks caps the grid with the chosen instantiation's own)
-    const int64_t resident_waves = int64_t(resident_blocks(device, precision, false)) * kWavesPerBlock;
-    const int chunk = int(std::max<int64_t>(1, std::min<int64_t>(launch_shape().chunk, src.n_tiles / resident_waves)));
-    const bool merge = src.n_tiles < kMergeDrainTiles * resident_waves;
-    const int64_t waves_needed = (src.n_tiles + chunk - 1) / chunk;
-    const unsigned grid = unsigned(std::max<int64_t>(1, std::min<int64_t>((waves_needed + kWavesPerBlock - 1) / kWavesPerBlock,
-                                                                          resident_blocks(device, precision, merge))));
-    const dim3 g3(grid), b3(kBlock);
-    if (precision == ADECO_PREC_FP64) {
-        if (merge)
-            hipLaunchKernelGGL((k_deposit_waves<ADECO_PREC_FP64, true>), g3, b3, 0, stream, src, chunk, queue_counter, counters);
-        else
-            hipLaunchKernelGGL((k_deposit_waves<ADECO_PREC_FP64, false>), g3, b3, 0, stream, src, chunk, queue_counter, counters);
-    } else if (precision == ADECO_PREC_MIXED) {
-        if (merge)
-            hipLaunchKernelGGL((k_deposit_waves<ADECO_PREC_MIXED, true>), g3, b3, 0, stream, src, chunk, queue_counter, counters);
-        else
-            hipLaunchKernelGGL((k_deposit_waves<ADECO_PREC_MIXED, false>), g3, b3, 0, stream, src, chunk, queue_counter, counters);
-    } else {
-        if (merge)
-            hipLaunchKernelGGL((k_deposit_waves<ADECO_PREC_FP32, true>), g3, b3, 0, stream, src, chunk, queue_counter, counters);
-        else
-            hipLaunchKernelGGL((k_deposit_waves<ADECO_PREC_FP32, false>), g3, b3, 0, stream, src, chunk, queue_counter, counters);
+    if (src.form == kFormBlocks) return launch_block_tiles(stream, src, queue_counter, counters, device);
+    const WaveLaunch w = wave_launch(src.n_tiles, deposit_occupancy(src.form, false), kWavesPerBlock, device);
+    // (the merged-drain instantiation's own occupancy is the same or lower)
+    const dim3 g3(w.merge ? std::min(w.grid, wave_launch(src.n_tiles, deposit_occupancy(src.form, true), kWavesPerBlock, device).grid)
+                          : w.grid);
+    const dim3 b3(kBlock);
+    switch (src.form * 2 + int(w.merge)) {
+        case 2 * kFormFp64: hipLaunchKernelGGL((k_deposit_waves<ADECO_PREC_FP64, false>), g3, b3, 0, stream, src, w.chunk, queue_counter, counters); break;
+        case 2 * kFormFp64 + 1: hipLaunchKernelGGL((k_deposit_waves<ADECO_PREC_FP64, true>), g3, b3, 0, stream, src, w.chunk, queue_counter, counters); break;
+        case 2 * kFormMixed: hipLaunchKernelGGL((k_deposit_waves<ADECO_PREC_MIXED, false>), g3, b3, 0, stream, src, w.chunk, queue_counter, counters); break;
+        case 2 * kFormMixed + 1: hipLaunchKernelGGL((k_deposit_waves<ADECO_PREC_MIXED, true>), g3, b3, 0, stream, src, w.chunk, queue_counter, counters); break;
+        case 2 * kFormFp32: hipLaunchKernelGGL((k_deposit_waves<ADECO_PREC_FP32, false>), g3, b3, 0, stream, src, w.chunk, queue_counter, counters); break;
+        default: hipLaunchKernelGGL((k_deposit_waves<ADECO_PREC_FP32, true>), g3, b3, 0, stream, src, w.chunk, queue_counter, counters); break;
     }
     return hipGetLastError();
 }
 
-hipError_t launch_deposit_step(hipStream_t stream, int precision, const TileSource* d_sources, const int2* d_entries,
+hipError_t launch_deposit_step(hipStream_t stream, int form, const TileSource* d_sources, const int2* d_entries,
                                int n_entries, unsigned* queue_counter, unsigned long long* counters, int device) {
     if (n_entries <= 0) return hipSuccess;
-    // small steps as small launches (launch_deposit_tiles)
-    const int64_t resident_waves = int64_t(resident_blocks(device, precision, false)) * kWavesPerBlock;
-    const int chunk = int(std::max<int64_t>(1, std::min<int64_t>(launch_shape().chunk, n_entries / resident_waves)));
-    const bool merge = n_entries < kMergeDrainTiles * resident_waves;
-    const int64_t waves_needed = (int64_t(n_entries) + chunk - 1) / chunk;
-    const unsigned grid = unsigned(std::max<int64_t>(1, std::min<int64_t>((waves_needed + kWavesPerBlock - 1) / kWavesPerBlock,
-                                                                          resident_blocks(device, precision, merge))));
-    const dim3 g3(grid), b3(kBlock);
-    if (precision == ADECO_PREC_FP64) {
-        if (merge)
-            hipLaunchKernelGGL((k_deposit_step<ADECO_PREC_FP64, true>), g3, b3, 0, stream, d_sources, d_entries, n_entries,
-                               chunk, queue_counter, counters);
-        else
-            hipLaunchKernelGGL((k_deposit_step<ADECO_PREC_FP64, false>), g3, b3, 0, stream, d_sources, d_entries, n_entries,
-                               chunk, queue_counter, counters);
-    } else if (precision == ADECO_PREC_MIXED) {
-        if (merge)
-            hipLaunchKernelGGL((k_deposit_step<ADECO_PREC_MIXED, true>), g3, b3, 0, stream, d_sources, d_entries, n_entries,
-                               chunk, queue_counter, counters);
-        else
-            hipLaunchKernelGGL((k_deposit_step<ADECO_PREC_MIXED, false>), g3, b3, 0, stream, d_sources, d_entries, n_entries,
-                               chunk, queue_counter, counters);
-    } else {
-        if (merge)
-            hipLaunchKernelGGL((k_deposit_step<ADECO_PREC_FP32, true>), g3, b3, 0, stream, d_sources, d_entries, n_entries,
-                               chunk, queue_counter, counters);
-        else
-            hipLaunchKernelGGL((k_deposit_step<ADECO_PREC_FP32, false>), g3, b3, 0, stream, d_sources, d_entries, n_entries,
-                               chunk, queue_counter, counters);
+    if (form == kFormBlocks) return launch_block_step(stream, d_sources, d_entries, n_entries, queue_counter, counters, device);
+    const WaveLaunch w = wave_launch(n_entries, deposit_occupancy(form, false), kWavesPerBlock, device);
+    const dim3 g3(w.merge ? std::min(w.grid, wave_launch(n_entries, deposit_occupancy(form, true), kWavesPerBlock, device).grid) : w.grid);
+    const dim3 b3(kBlock);
+    switch (form * 2 + int(w.merge)) {
+        case 2 * kFormFp64: hipLaunchKernelGGL((k_deposit_step<ADECO_PREC_FP64, false>), g3, b3, 0, stream, d_sources, d_entries, n_entries, w.chunk, queue_counter, counters); break;
+        case 2 * kFormFp64 + 1: hipLaunchKernelGGL((k_deposit_step<ADECO_PREC_FP64, true>), g3, b3, 0, stream, d_sources, d_entries, n_entries, w.chunk, queue_counter, counters); break;
+        case 2 * kFormMixed: hipLaunchKernelGGL((k_deposit_step<ADECO_PREC_MIXED, false>), g3, b3, 0, stream, d_sources, d_entries, n_entries, w.chunk, queue_counter, counters); break;
+        case 2 * kFormMixed + 1: hipLaunchKernelGGL((k_deposit_step<ADECO_PREC_MIXED, true>), g3, b3, 0, stream, d_sources, d_entries, n_entries, w.chunk, queue_counter, counters); break;
+        case 2 * kFormFp32: hipLaunchKernelGGL((k_deposit_step<ADECO_PREC_FP32, false>), g3, b3, 0, stream, d_sources, d_entries, n_entries, w.chunk, queue_counter, counters); break;
+        default: hipLaunchKernelGGL((k_deposit_step<ADECO_PREC_FP32, true>), g3, b3, 0, stream, d_sources, d_entries, n_entries, w.chunk, queue_counter, counters); break;
     }
     return hipGetLastError();
 }
@@ -1108,13 +1019,14 @@ adeco_status prepare_leaves_batched(adeco_octree_s* T, hipStream_t stream, int d
     const LatticeView lv{L->d_x, L->d_y, L->d_z, {L->np[0], L->np[1], L->np[2]}};
     const PackedCorners ct = pack_corners(corner_table(decomposition));
     CandidateSpace cs;
+    const int form = deposit_form(precision, gd.data(), nl);
     // (synchronises the stream, so gd may go out of scope afterwards)
     if ((st = build_candidate_space(stream, lv, ct, T->d_pairs.as<int32_t>(), P, T->d_leaf_offset.as<int64_t>(), nl,
-                                    geom.as<GridDesc>(), tet_mass, precision, work.ptr, cs)))
+                                    geom.as<GridDesc>(), tet_mass, form, work.ptr, cs)))
         return st;
     if ((st = tiles.reserve(tile_map_bytes(cs.n_cand)))) return st;
     if ((st = build_tile_map(stream, cs, tiles.as<int32_t>()))) return st;
-    src = TileSource{cs.pd, cs.cand_off, cs.tile_first, cs.n_tiles, cs.n_cand, geom.as<GridDesc>(), grids, tet_mass};
+    src = TileSource{cs.pd, cs.cand_off, cs.tile_first, cs.n_tiles, cs.n_cand, geom.as<GridDesc>(), grids, tet_mass, form};
     return ADECO_OK;
 }
 
@@ -1133,7 +1045,7 @@ adeco_status deposit_leaves_batched(adeco_octree_s* T, int dims, int decompositi
     hipError_t e = hipMemsetAsync(T->d_counters.ptr, 0, 64, ds.stream);
     if (e != hipSuccess) return hip_fail(e, "batched counters");
     e = hipEventRecord(ds.evk0, ds.stream);
-    if (e == hipSuccess) e = launch_deposit_tiles(ds.stream, precision, src, ctr, counters, L->device);
+    if (e == hipSuccess) e = launch_deposit_tiles(ds.stream, src, ctr, counters, L->device);
     if (e == hipSuccess) e = hipEventRecord(ds.evk1, ds.stream);
     if (e != hipSuccess) return hip_fail(e, "batched deposit launch");
     T->last_candidates = src.n_cand;

@@ -19,6 +19,11 @@ constexpr int kWaveTile = 64;  // candidates per tile == lanes per wavefront
 // deposits use single cells.
 constexpr int kMaxSeg = 8;
 
+// Form of a candidate space and of the kernel that deposits it: the column and single-cell forms by
+// precision (batched.hip), or cell blocks (blocks.hip), the FP64 form wherever every grid has unit
+// scaled cells.
+enum DepositForm : int { kFormFp64 = ADECO_PREC_FP64, kFormMixed = ADECO_PREC_MIXED, kFormFp32 = ADECO_PREC_FP32, kFormBlocks = 3 };
+
 // One output grid: a leaf or a request ROI.  gmin/delta/scale in FP64; base = first cell of the
 // grid in the grid buffer; cells i + dims*(j + dims*k).
 struct GridDesc {
@@ -34,8 +39,12 @@ struct GridDesc {
 
 GridDesc make_grid_desc(const GridGeom& g, long long base);
 
+// The form of a deposit of the given precision onto n grids.
+int deposit_form(int precision, const GridDesc* grids, int64_t n);
+
 // Everything the deposit needs about one binned (grid, tet) pair, written once by the pair setup:
-// one 128-byte line per pair.
+// one 128-byte line per pair.  In the block form the vertices and the range are in the pair's own axis
+// order (x, y, z: from the shortest to the longest covered extent), bits 60-62 of the range.
 struct alignas(128) PairData {
     double S[12];              // scale_a * (v_q - gmin_a), vertices in the oriented order
     double mcell;              // tet_mass * cell_vol / |V|
@@ -56,6 +65,7 @@ struct TileSource {
     const GridDesc* grids;
     double* grid_buf;
     double tet_mass;
+    int form = 0;                        // DepositForm
     const int64_t* dev_sizes = nullptr;  // when set, n_cand and n_tiles are dev_sizes[0], [1] (device)
 };
 
@@ -68,6 +78,7 @@ struct CandidateSpace {
     int64_t* total = nullptr;
     int32_t* tile_first = nullptr;
     int64_t n_pairs = 0, n_cand = 0, n_tiles = 0;
+    int form = 0;
 };
 
 // Launch shape of the persistent deposit: tiles taken per work-queue pop and resident workgroups
@@ -79,9 +90,9 @@ struct LaunchShape {
     int blocks_per_cu = 4;
 };
 LaunchShape& launch_shape();
-// Workgroups of the persistent deposit kernel (precision, merged drain or not) that one CU holds at
+// Workgroups of the persistent deposit kernel (form, merged drain or not) that one CU holds at
 // once (hipOccupancyMaxActiveBlocksPerMultiprocessor on the current device); at least 1.
-int deposit_occupancy(int precision, bool merge);
+int deposit_occupancy(int form, bool merge);
 
 // Bytes of the work slab for n_pairs pairs (tile map excluded: it needs n_cand).
 size_t candidate_space_bytes(int64_t n_pairs);
@@ -89,11 +100,11 @@ size_t tile_map_bytes(int64_t n_cand);
 
 // Lays out `cs` in `slab` and runs pair setup + scan (asynchronous; n_cand is read back with a
 // synchronous copy).  Pairs are grid-major: grid_off is the CSR offset of each grid's pairs.
-// precision selects the candidate unit: column segments for ADECO_PREC_FP64 on grids with unit
-// scaled cells, single cells otherwise.
+// form (deposit_form) selects the candidate unit: cell blocks, column segments (FP64, on the grids with
+// unit scaled cells) or single cells.
 adeco_status build_candidate_space(hipStream_t stream, const LatticeView& lat, const PackedCorners& ct,
                                    const int32_t* pairs, int64_t n_pairs, const int64_t* grid_off, int n_grids,
-                                   const GridDesc* d_grids, double tet_mass, int precision, void* slab,
+                                   const GridDesc* d_grids, double tet_mass, int form, void* slab,
                                    CandidateSpace& cs);
 // Writes the tile map into `tiles` (tile_map_bytes(cs.n_cand) bytes).
 adeco_status build_tile_map(hipStream_t stream, CandidateSpace& cs, int32_t* tiles);
@@ -105,7 +116,7 @@ adeco_status build_tile_map(hipStream_t stream, CandidateSpace& cs, int32_t* til
 hipError_t enqueue_candidate_space_dev(hipStream_t stream, const LatticeView& lat, const PackedCorners& ct,
                                        const int32_t* pairs, int64_t pair_cap, const int64_t* n_dev,
                                        const int64_t* grid_off, int n_grids, const GridDesc* d_grids, double tet_mass,
-                                       int precision, void* slab, int32_t* tiles, int64_t tile_cap, int64_t* sizes,
+                                       int form, void* slab, int32_t* tiles, int64_t tile_cap, int64_t* sizes,
                                        unsigned* overflow, CandidateSpace& cs);
 
 // Exclusive scan of n uint32 counts into int64 offsets out[0..n] (out[n] = the total); block_sum
@@ -114,13 +125,13 @@ hipError_t launch_scan_u32(const unsigned* in, int64_t n, int64_t* out, int64_t*
                            hipStream_t stream);
 size_t scan_block_words(int64_t n);
 
-// Persistent deposit over one candidate space (built for the same precision); counters[0] += exact
-// recomputes, counters[1] += partial candidates.  queue_counter must be zero.
-hipError_t launch_deposit_tiles(hipStream_t stream, int precision, const TileSource& src, unsigned* queue_counter,
+// Persistent deposit over one candidate space (src.form); counters[0] += exact recomputes,
+// counters[1] += partial candidates.  queue_counter must be zero.
+hipError_t launch_deposit_tiles(hipStream_t stream, const TileSource& src, unsigned* queue_counter,
                                 unsigned long long* counters, int device);
 
-// One serving step: entries (source slot, tile) over several candidate spaces in one launch.
-hipError_t launch_deposit_step(hipStream_t stream, int precision, const TileSource* d_sources,
+// One serving step: entries (source slot, tile) over several candidate spaces of one form in one launch.
+hipError_t launch_deposit_step(hipStream_t stream, int form, const TileSource* d_sources,
                                const int2* d_entries, int n_entries, unsigned* queue_counter,
                                unsigned long long* counters, int device);
 
@@ -129,6 +140,27 @@ hipError_t launch_deposit_step(hipStream_t stream, int precision, const TileSour
 adeco_status prepare_leaves_batched(adeco_octree_s* T, hipStream_t stream, int dims, int decomposition, double tet_mass,
                                     int precision, DevBuf& geom, DevBuf& work, DevBuf& tiles, double* grids,
                                     TileSource& src);
+
+// The block form's kernels (blocks.hip).
+hipError_t launch_block_setup(hipStream_t stream, const LatticeView& lat, const PackedCorners& ct, const int32_t* pairs,
+                              int64_t n_pairs, const int64_t* n_dev, const int64_t* grid_off, int n_grids,
+                              const int32_t* pair_grid, const GridDesc* d_grids, double tet_mass, unsigned* cand, PairData* pd);
+int block_occupancy();
+hipError_t launch_block_tiles(hipStream_t stream, const TileSource& src, unsigned* queue_counter,
+                              unsigned long long* counters, int device);
+hipError_t launch_block_step(hipStream_t stream, const TileSource* d_sources, const int2* d_entries, int n_entries,
+                             unsigned* queue_counter, unsigned long long* counters, int device);
+
+// Launch of a persistent kernel over n_items tiles with `occupancy` workgroups of `waves` wavefronts
+// resident per CU.  Launches with fewer than kMergeDrainTiles tiles per resident wave are small: tiles per
+// pop so that every wave gets some, and drain passes merged across the work classes.
+constexpr int64_t kMergeDrainTiles = 16;
+struct WaveLaunch {
+    unsigned grid;
+    int chunk;
+    bool merge;
+};
+WaveLaunch wave_launch(int64_t n_items, int occupancy, int waves, int device);
 
 // Clears n 32-bit words with a kernel (a memset node in a captured graph is avoided).
 hipError_t launch_zero_u32(unsigned* p, int n, hipStream_t stream);

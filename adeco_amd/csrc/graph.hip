@@ -88,7 +88,7 @@ adeco_status adeco_deposit_graph_create(adeco_octree T, int dims, int decomposit
     e = hipStreamBeginCapture(G->stream, hipStreamCaptureModeThreadLocal);
     if (e == hipSuccess) e = launch_fill_f64(G->grids.as<double>(), words, 0.0, G->stream);
     if (e == hipSuccess) e = launch_zero_u32(ctr, 16, G->stream);
-    if (e == hipSuccess) e = launch_deposit_tiles(G->stream, precision, G->src, ctr, counters, G->device);
+    if (e == hipSuccess) e = launch_deposit_tiles(G->stream, G->src, ctr, counters, G->device);
     hipGraph_t graph = nullptr;
     const hipError_t ec = hipStreamEndCapture(G->stream, &graph);
     G->graph = graph;
@@ -222,7 +222,7 @@ adeco_status adeco_deposit_graph_create_step(adeco_octree T, int dims, int decom
     unsigned* ctr = G->counters.as<unsigned>();
     unsigned long long* counters = reinterpret_cast<unsigned long long*>(G->counters.as<char>() + 16);
     int64_t* sizes = G->b_sizes.as<int64_t>();
-    G->src = TileSource{nullptr, nullptr, nullptr, G->tile_cap, 0, G->geom.as<GridDesc>(), G->grids.as<double>(), tet_mass};
+    G->src = TileSource{nullptr, nullptr, nullptr, G->tile_cap, 0, G->geom.as<GridDesc>(), G->grids.as<double>(), tet_mass, eager.form};
     e = hipStreamBeginCapture(G->stream, hipStreamCaptureModeThreadLocal);
     if (e == hipSuccess) e = launch_zero_u32(ctr, 16, G->stream);  // queue counter and overflow flag
     if (e == hipSuccess) e = bin_count_async(plan, G->stream);
@@ -232,7 +232,7 @@ adeco_status adeco_deposit_graph_create_step(adeco_octree T, int dims, int decom
     CandidateSpace cs;
     if (e == hipSuccess)
         e = enqueue_candidate_space_dev(G->stream, lv, plan.ct, G->b_pairs.as<int32_t>(), G->pair_cap, n_pairs_dev,
-                                        leaf_offset, int(nl), G->geom.as<GridDesc>(), tet_mass, precision, G->work.ptr,
+                                        leaf_offset, int(nl), G->geom.as<GridDesc>(), tet_mass, eager.form, G->work.ptr,
                                         G->tiles.as<int32_t>(), G->tile_cap, sizes, ctr + 1, cs);
     if (e == hipSuccess) {
         G->src.pd = cs.pd;
@@ -245,7 +245,7 @@ adeco_status adeco_deposit_graph_create_step(adeco_octree T, int dims, int decom
     // (the launch shape is chosen from the capture's tile count; the kernel reads the replay's)
     TileSource shape = G->src;
     shape.n_tiles = eager.n_tiles;
-    if (e == hipSuccess) e = launch_deposit_tiles(G->stream, precision, shape, ctr, counters, G->device);
+    if (e == hipSuccess) e = launch_deposit_tiles(G->stream, shape, ctr, counters, G->device);
     hipGraph_t graph = nullptr;
     const hipError_t ec = hipStreamEndCapture(G->stream, &graph);
     G->graph = graph;

@@ -107,16 +107,16 @@ adeco_status deposit_soup_batched(DeviceState& ds, const float* d_tets, int64_t 
     LatticeView lv{nullptr, nullptr, nullptr, {0, 0, 0}, d_tets};
     const PackedCorners ct = pack_corners(corner_table(0));
     CandidateSpace cs;
-    if ((st = build_candidate_space(ds.stream, lv, ct, ids.as<int32_t>(), n_tets, d_goff, 1, d_gd, tet_mass, precision,
-                                    work.ptr, cs)))
+    if ((st = build_candidate_space(ds.stream, lv, ct, ids.as<int32_t>(), n_tets, d_goff, 1, d_gd, tet_mass,
+                                    deposit_form(precision, &gd, 1), work.ptr, cs)))
         return st;
     if ((st = tiles.reserve(tile_map_bytes(cs.n_cand))) || (st = build_tile_map(ds.stream, cs, tiles.as<int32_t>()))) return st;
     unsigned* q = ctr.as<unsigned>();
     unsigned long long* counters = reinterpret_cast<unsigned long long*>(ctr.as<char>() + 16);
     e = launch_zero_u32(q, 16, ds.stream);
-    const TileSource src{cs.pd, cs.cand_off, cs.tile_first, cs.n_tiles, cs.n_cand, d_gd, d_grid, tet_mass};
+    const TileSource src{cs.pd, cs.cand_off, cs.tile_first, cs.n_tiles, cs.n_cand, d_gd, d_grid, tet_mass, cs.form};
     if (e == hipSuccess) e = hipEventRecord(ds.evk0, ds.stream);
-    if (e == hipSuccess) e = launch_deposit_tiles(ds.stream, precision, src, q, counters, ds.id);
+    if (e == hipSuccess) e = launch_deposit_tiles(ds.stream, src, q, counters, ds.id);
     if (e == hipSuccess) e = hipEventRecord(ds.evk1, ds.stream);
     unsigned long long cnt[2] = {0, 0};
     if (e == hipSuccess) e = hipMemcpyAsync(cnt, counters, 16, hipMemcpyDeviceToHost, ds.stream);

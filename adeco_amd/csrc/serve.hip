@@ -289,6 +289,7 @@ struct adeco_server_s {
         float* host_out = nullptr;
         int slot = -1;
         int64_t n_tets = 0, n_cand = 0, n_tiles = 0, next_tile = 0;
+        int form = 0;  // of its candidate space
         double t_submit = 0, t_admit = -1, t_done = -1;
         adeco_status status = ADECO_OK;
         bool done = false;
@@ -425,14 +426,15 @@ adeco_status adeco_server_s::admit(Req* r, int si) {
     if (r->n_tets > 0) {
         CandidateSpace cs;
         if ((st = build_candidate_space(admit_stream, lv, ct, s.pairs.as<int32_t>(), r->n_tets, d_goff, 1, d_gd, cfg.tet_mass,
-                                        cfg.precision, s.work.ptr, cs)))
+                                        deposit_form(cfg.precision, &r->gd, 1), s.work.ptr, cs)))
             return st;
         if ((st = s.tiles.reserve(tile_map_bytes(cs.n_cand)))) return st;
         if ((st = build_tile_map(admit_stream, cs, s.tiles.as<int32_t>()))) return st;
         r->n_cand = cs.n_cand;
         r->n_tiles = cs.n_tiles;
+        r->form = cs.form;
         h_sources[si] = TileSource{cs.pd, cs.cand_off, cs.tile_first, cs.n_tiles, cs.n_cand, d_gd, s.grid.as<double>(),
-                                   cfg.tet_mass};
+                                   cfg.tet_mass, cs.form};
         e = hipMemcpyAsync(d_sources.as<TileSource>() + si, &h_sources[si], sizeof(TileSource), hipMemcpyHostToDevice,
                            admit_stream);
         if (e != hipSuccess) return hip_fail(e, "request setup");
@@ -529,7 +531,9 @@ void adeco_server_s::run_worker() {
         }
         int2* he = h_entries[buf];
         const int64_t cap = cfg.step_tiles;
-        int n = 0;
+        // entries of block-form requests from the front of the buffer, the others' (another precision, or
+        // admitted under the reference's cell scaling) from its end: one launch for each form
+        int n = 0, n_front = 0;
         int64_t left = cap;
         size_t open = 0;
         for (Req* r : run) open += r->next_tile < r->n_tiles ? 1 : 0;
@@ -540,7 +544,11 @@ void adeco_server_s::run_worker() {
                 const int64_t rem = r->n_tiles - r->next_tile;
                 if (rem <= 0 || left <= 0) continue;
                 const int64_t take = std::min(std::min(rem, quota), left);
-                for (int64_t t = 0; t < take; ++t) he[n++] = make_int2(r->slot, int(r->next_tile + t));
+                const bool front = r->form == kFormBlocks;
+                int2* at = front ? he + n_front : he + cap - (n - n_front) - take;
+                for (int64_t t = 0; t < take; ++t) at[t] = make_int2(r->slot, int(r->next_tile + t));
+                n += int(take);
+                n_front += front ? int(take) : 0;
                 r->next_tile += take;
                 left -= take;
                 if (r->next_tile < r->n_tiles) ++open;
@@ -549,7 +557,11 @@ void adeco_server_s::run_worker() {
         unsigned* ctr = d_ctr.as<unsigned>();
         unsigned long long* counters = reinterpret_cast<unsigned long long*>(d_ctr.as<char>() + 16);
         if (n > 0 && e == hipSuccess) {
-            e = hipMemcpyAsync(d_entries[buf].ptr, he, size_t(n) * sizeof(int2), hipMemcpyHostToDevice, stream);
+            const int n_back = n - n_front;
+            int2* de = d_entries[buf].as<int2>();
+            if (n_front) e = hipMemcpyAsync(de, he, size_t(n_front) * sizeof(int2), hipMemcpyHostToDevice, stream);
+            if (n_back && e == hipSuccess)
+                e = hipMemcpyAsync(de + cap - n_back, he + cap - n_back, size_t(n_back) * sizeof(int2), hipMemcpyHostToDevice, stream);
             if (e == hipSuccess) e = hipEventRecord(entries_uploaded[buf], stream);
             if (e == hipSuccess) entries_in_flight[buf] = true;
             if (e == hipSuccess) e = launch_zero_u32(ctr, 16, stream);
@@ -568,7 +580,9 @@ void adeco_server_s::run_worker() {
             }
             if (e == hipSuccess) e = hipEventRecord(ev.first, stream);
             if (e == hipSuccess)
-                e = launch_deposit_step(stream, cfg.precision, d_sources.as<TileSource>(), d_entries[buf].as<int2>(), n, ctr,
+                e = launch_deposit_step(stream, kFormBlocks, d_sources.as<TileSource>(), de, n_front, ctr, counters, L->device);
+            if (e == hipSuccess)
+                e = launch_deposit_step(stream, cfg.precision, d_sources.as<TileSource>(), de + cap - n_back, n_back, ctr + 1,
                                         counters, L->device);
             if (e == hipSuccess) e = hipEventRecord(ev.second, stream);
             lk.lock();

@@ -410,7 +410,7 @@ adeco_status adeco_autotune_batched(adeco_octree T, int dims, int decomposition,
     {
         std::lock_guard<std::mutex> lk(T->L->ds->mutex);
         if (hipSetDevice(T->L->device) != hipSuccess) return fail(ADECO_EDEVICE, "autotune_batched(): hipSetDevice failed");
-        max_blocks = std::min(4, deposit_occupancy(precision, false));
+        max_blocks = std::min(4, deposit_occupancy(precision == ADECO_PREC_FP64 && cell_scaling() == kScalingExact ? int(kFormBlocks) : precision, false));
     }
     const LaunchShape saved = launch_shape();
     double best = 1e300;
