@@ -226,12 +226,6 @@ __global__ void __launch_bounds__(256) k_pair_grid(const int64_t* __restrict__ g
 // the one holding out[n_dev].)
 constexpr int kScanBlock = 1024;
 
-__device__ __forceinline__ int64_t shfl_up_i64(int64_t v, int d) {
-    const int lo = __shfl_up(int(uint64_t(v) & 0xffffffffu), d, 64);
-    const int hi = __shfl_up(int(uint64_t(v) >> 32), d, 64);
-    return int64_t((uint64_t(unsigned(hi)) << 32) | unsigned(lo));
-}
-
 __device__ __forceinline__ int64_t shfl_xor_i64(int64_t v, int m) {
     const int lo = __shfl_xor(int(uint64_t(v) & 0xffffffffu), m, 64);
     const int hi = __shfl_xor(int(uint64_t(v) >> 32), m, 64);

@@ -22,7 +22,7 @@
 
 namespace adeco {
 
-// Largest number of cells in a block.
+// Largest number of cells in a block (a kernel may take smaller ones).
 constexpr int kBlockCells = 16;
 // Shares of a cell below kNoShare (18 ulps of the tet: the differences' rounding) are empty; between
 // that and kSmallShare they are recomputed by exact_cell_share.
@@ -365,9 +365,14 @@ ADECO_HD double slab_share(const double z[4]) {
 
 // Share of the tet in the unit cell [0, 1]^3 from non-overlapping pieces: x >= 0, x <= 1, y >= 0,
 // y <= 1 in turn, then the z slab; all terms are positive.  keep(i), i < 15, is storage for the points of
-// the first cut, so that only the inner cuts' stay in registers.
+// the first cut, so that only the inner cuts' stay in registers.  The work can be shared out: of the 27
+// paths (one piece of each of the first three cuts) this call sums those with index `first`,
+// `first` + `stride`, ... (stride a power of 2).
 template <class Keep>
-ADECO_HD double exact_cell_share(const double x[4], const double y[4], const double z[4], Keep keep) {
+ADECO_HD double exact_cell_share(const double x[4], const double y[4], const double z[4], Keep keep, int first = 0,
+                                 int stride = 1) {
+    // whether any of the paths at..at + n - 1 is this call's
+    const auto mine = [&](int at, int n) { return ((first - at) & (stride - 1)) < n; };
     int count;
     double p0[3], w0, w1, w2;
     {
@@ -389,20 +394,23 @@ ADECO_HD double exact_cell_share(const double x[4], const double y[4], const dou
         w2 = a.w[2];
     }
     double sum = 0.0;
-    for (int ka = 0; ka < count; ++ka) {
+    for (int ka = 0;; ++ka) {
+        while (ka < count && !mine(9 * ka, 9)) ++ka;
+        if (ka >= count) break;
         double k2[4], v2[2][4];
-        k2[0] = p0[0];
-        v2[0][0] = p0[1];
-        v2[1][0] = p0[2];
-        for (int i = 1; i < 4; ++i) {
-            k2[i] = keep(3 * (ka + i - 1));
-            v2[0][i] = keep(3 * (ka + i - 1) + 1);
-            v2[1][i] = keep(3 * (ka + i - 1) + 2);
+        for (int i = 0; i < 4; ++i) {
+            const int at = 3 * (ka + i - 1);
+            const bool held = ka == 0 && i == 0;
+            k2[i] = held ? p0[0] : keep(held ? 0 : at);
+            v2[0][i] = held ? p0[1] : keep(held ? 0 : at + 1);
+            v2[1][i] = held ? p0[2] : keep(held ? 0 : at + 2);
         }
-        for (int m = 0; m < 3; ++m) p0[m] = keep(3 * ka + m);
+        const double wa = ka == 0 ? w0 : (ka == 1 ? w1 : w2);
         PositivePart<2> b;
         b.set(k2, v2);
-        for (int kb = 0; kb < b.count; ++kb) {
+        for (int kb = 0;; ++kb) {
+            for (; kb < b.count && !mine(9 * ka + 3 * kb, 3); ++kb) b.advance();
+            if (kb >= b.count) break;
             double v3[2][4];
             for (int i = 0; i < 4; ++i) {
                 v3[0][i] = 1.0 - b.s[0][i];
@@ -411,8 +419,10 @@ ADECO_HD double exact_cell_share(const double x[4], const double y[4], const dou
             const double k3[4] = {b.s[0][0], b.s[0][1], b.s[0][2], b.s[0][3]};
             PositivePart<2> c;
             c.set(k3, v3);
-            const double wb = w0 * b.w[0];
-            for (int kc = 0; kc < c.count; ++kc) {
+            const double wb = wa * b.w[0];
+            for (int kc = 0;; ++kc) {
+                for (; kc < c.count && !mine(9 * ka + 3 * kb + kc, 1); ++kc) c.advance();
+                if (kc >= c.count) break;
                 const double v4[1][4] = {{c.s[1][0], c.s[1][1], c.s[1][2], c.s[1][3]}};
                 const double k4[4] = {c.s[0][0], c.s[0][1], c.s[0][2], c.s[0][3]};
                 PositivePart<1> d;
@@ -427,8 +437,6 @@ ADECO_HD double exact_cell_share(const double x[4], const double y[4], const dou
             }
             b.advance();
         }
-        w0 = w1;
-        w1 = w2;
     }
     return sum;
 }

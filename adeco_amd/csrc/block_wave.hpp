@@ -1,0 +1,408 @@
+// Wavefront machinery of the block deposits (blocks.hip, direct.hip): how a tet's covered cells are cut
+// into blocks, the per-wave work queues, and the loop that clips them.
+//
+// A block to clip is queued by its work class and a queue that holds 64 of them is clipped by the
+// whole wave, each lane summing one block's shares in its own LDS column.  A cell whose share is small
+// against the rounding of the differences goes to one more queue, whose passes recompute it alone.
+#pragma once
+
+#include <hip/hip_runtime.h>
+
+#include "batched_impl.hpp"
+#include "block_clip.hpp"
+#include "wave_tiles.hpp"
+
+namespace adeco {
+
+constexpr int kClasses = 6;            // queues of blocks to clip
+constexpr int kExact = kClasses;       // the queue of single cells to recompute
+constexpr int kQueues = kClasses + 1;
+
+// Per-wavefront LDS for blocks of up to E cells.  A queue entry is an int2 that the kernel's loader
+// understands.  An entry that finds its queue full is carried per lane and takes its place once that
+// queue has been clipped; qn[b] counts queue b's entries and its carried ones.
+template <int E>
+struct BlockLds {
+    static_assert(E >= 15, "exact_cell_share keeps 15 values in a lane's column");
+    int qn[16];
+    int2 q[kQueues][kWaveTile];
+    int2 carry[kWaveTile];
+    signed char carry_key[kWaveTile];
+    unsigned char cell[kWaveTile];  // of each exact-queue entry
+    union {
+        double acc[E][kWaveTile];  // each lane's shares
+        int mark[kWaveTile];       // starts of the tile being classified
+    };
+};
+
+// How covered cells are cut into blocks: blocks of b cells, n of them, per axis (x, y, z in the pair's
+// order, extents ex <= ey <= ez).  A cover of at most E cells is one block; else x keeps up to 2 cells, z
+// up to 4 (3 of E = 12) and y what is left, the cells spread evenly over an axis' blocks.
+struct BlockShape {
+    int b[3], n[3];
+};
+
+template <int E>
+__device__ __forceinline__ BlockShape block_shape(int ex, int ey, int ez) {
+    static_assert(E == 12 || E == 16, "block sizes");
+    BlockShape s;
+    s.b[0] = ex;
+    s.b[1] = ey;
+    s.b[2] = ez;
+    s.n[0] = s.n[1] = s.n[2] = 1;
+    if (ex * ey * ez <= E) return s;
+    const int bz = min(ez, E / 4);
+    const int bx = min(ex, 2), xz = bx * bz;
+    // E / (bx * bz) for the products that occur (1-4, 6, 8)
+    const int room = E == 16 ? (xz <= 2 ? 8 : (xz == 3 ? 5 : (xz == 4 ? 4 : 2))) : (xz <= 2 ? 6 : (xz == 3 ? 4 : (xz == 4 ? 3 : 2)));
+    const int b[3] = {bx, min(ey, room), bz};
+    for (int a = 0; a < 3; ++a)
+        if (b[a] < s.b[a]) {
+            const int e = s.b[a], n = int(udiv_small(unsigned(e + b[a] - 1), unsigned(b[a])));
+            s.b[a] = int(udiv_small(unsigned(e + n - 1), unsigned(n)));
+            s.n[a] = int(udiv_small(unsigned(e + s.b[a] - 1), unsigned(s.b[a])));
+        }
+    return s;
+}
+
+// Axis order of a cover, packed in 3 bits: the axis of z and whether x and y are the next two axes in
+// cyclic order or the reverse.
+__device__ __forceinline__ int role_axis(int code, int role) {
+    const int za = code & 3, u = za == 2 ? 0 : za + 1, v = u == 2 ? 0 : u + 1;
+    const bool swap = code & 4;
+    return role == 2 ? za : ((role == 0) != swap ? u : v);
+}
+
+template <class T>
+__device__ __forceinline__ T pick(int a, T v0, T v1, T v2) {
+    return a == 0 ? v0 : (a == 1 ? v1 : v2);
+}
+
+// The order of the axes for extents e: z the longest (ties: z, then y), x the shorter of the others.
+__device__ __forceinline__ int role_code(const int e[3]) {
+    const int za = e[2] >= e[1] && e[2] >= e[0] ? 2 : (e[1] >= e[0] ? 1 : 0);
+    const int u = za == 2 ? 0 : za + 1, w = u == 2 ? 0 : u + 1;
+    return za | (pick(w, e[0], e[1], e[2]) < pick(u, e[0], e[1], e[2]) ? 4 : 0);
+}
+
+// Covered cells l..h of one axis for a tet between mn and mx (in cells from the grid's face): the cells
+// whose box it can strictly overlap, widened by 1e-9 of a cell and kept inside the grid.
+__device__ __forceinline__ void covered(double mn, double mx, int dims, int& l, int& h) {
+    const double top = double(dims - 1);
+    l = int(fmax(fmin(floor(mn - 1e-9), top), 0.0));
+    h = int(fmax(fmin(floor(mx + 1e-9), top), 0.0));
+}
+
+// A block of a cover: its corner cell (in the cover's axis order), its sizes and the tet's vertices from
+// the corner.
+struct Block {
+    int lo[3], c[3];
+    double x[4], y[4], z[4];
+};
+
+// lo, e: the cover's first cell and extents in its axis order; s: the vertices in cells, in that order.
+template <int E>
+__device__ __forceinline__ Block make_block(const int lo[3], const int e[3], const double s[4][3], unsigned unit) {
+    Block b;
+    const BlockShape sh = block_shape<E>(e[0], e[1], e[2]);
+    int i[3] = {0, 0, 0};
+    if (unit) {
+        const unsigned rest = sh.n[2] == 1 ? unit : udiv_small(unit, unsigned(sh.n[2]));
+        i[2] = int(unit - rest * unsigned(sh.n[2]));
+        i[0] = sh.n[1] == 1 ? int(rest) : int(udiv_small(rest, unsigned(sh.n[1])));
+        i[1] = int(rest) - i[0] * sh.n[1];
+    }
+    for (int a = 0; a < 3; ++a) {
+        b.lo[a] = lo[a] + i[a] * sh.b[a];
+        b.c[a] = min(sh.b[a], e[a] - i[a] * sh.b[a]);
+    }
+    for (int q = 0; q < 4; ++q) {
+        b.x[q] = s[q][0] - double(b.lo[0]);
+        b.y[q] = s[q][1] - double(b.lo[1]);
+        b.z[q] = s[q][2] - double(b.lo[2]);
+    }
+    return b;
+}
+
+// Where a block's cells lie: the offset of its first cell and the strides of its axes.
+struct Place {
+    int64_t corner, sx, sy, sz;
+};
+
+__device__ __forceinline__ Place place_of(const int lo[3], int code, int dims) {
+    const int64_t s1 = dims, s2 = int64_t(dims) * dims;
+    Place p;
+    p.sx = pick(role_axis(code, 0), int64_t(1), s1, s2);
+    p.sy = pick(role_axis(code, 1), int64_t(1), s1, s2);
+    p.sz = pick(role_axis(code, 2), int64_t(1), s1, s2);
+    p.corner = lo[0] * p.sx + lo[1] * p.sy + lo[2] * p.sz;
+    return p;
+}
+
+// Visits the cells of a block in the order of its shares: f(index, offset in the grid).
+template <class F>
+__device__ __forceinline__ void for_cells(const int c[3], const Place& p, F f) {
+    const int n = c[0] * c[1] * c[2];
+    int b = 0, k = 0;
+    int64_t at = p.corner;
+    const int64_t next_y = p.sy - c[2] * p.sz, next_x = p.sx - c[1] * p.sy;
+    for (int i = 0; i < n; ++i) {
+        f(i, at);
+        at += p.sz;
+        if (++k == c[2]) {
+            k = 0;
+            at += next_y;
+            if (++b == c[1]) {
+                b = 0;
+                at += next_x;
+            }
+        }
+    }
+}
+
+// Work class of a block to clip: by the planes that cut the tet across x and y, and for a single x plane
+// by whether it leaves one piece (1 or 3 vertices below) or three.  The class only groups blocks of
+// similar loops.  mn, mx: the tet's extents from the block's corner.
+__device__ __forceinline__ int work_class(const Block& b, const double mn[3], const double mx[3]) {
+    const int fx = floor_clamped(mn[0], b.c[0]) + 1, lx = min(ceil_clamped(mx[0], b.c[0]) - 1, b.c[0]);
+    const int fy = floor_clamped(mn[1], b.c[1]) + 1, ly = min(ceil_clamped(mx[1], b.c[1]) - 1, b.c[1]);
+    const int px = lx - fx + 1, py = ly - fy + 1;
+    if (px <= 0) return 0;
+    if (px >= 2) return 5;
+    int n = 0;
+    for (int q = 0; q < 4; ++q) n += int(b.x[q] < double(fx));
+    return (py <= 1 ? 1 : 3) + int(n == 2);
+}
+
+enum BlockClass : int { kBlockEmpty = -1, kBlockTet = -2, kBlockFull = -3 };
+
+// What to do with a block: nothing, deposit the whole tet in its only cell, fill it, or clip it (the work
+// class >= 0).  The tet is positively oriented in the block's axis order.
+__device__ __forceinline__ int classify_block(const Block& b) {
+    const double mn[3] = {fmin(fmin(b.x[0], b.x[1]), fmin(b.x[2], b.x[3])), fmin(fmin(b.y[0], b.y[1]), fmin(b.y[2], b.y[3])),
+                          fmin(fmin(b.z[0], b.z[1]), fmin(b.z[2], b.z[3]))};
+    const double mx[3] = {fmax(fmax(b.x[0], b.x[1]), fmax(b.x[2], b.x[3])), fmax(fmax(b.y[0], b.y[1]), fmax(b.y[2], b.y[3])),
+                          fmax(fmax(b.z[0], b.z[1]), fmax(b.z[2], b.z[3]))};
+    const double box[3] = {double(b.c[0]), double(b.c[1]), double(b.c[2])};
+    bool hit = true, inside = true;
+    for (int a = 0; a < 3; ++a) {
+        hit = hit && mn[a] < box[a] && 0.0 < mx[a];
+        inside = inside && mn[a] >= 0.0 && mx[a] <= box[a];
+    }
+    if (!hit) return kBlockEmpty;
+    if (inside) {
+        if (b.c[0] * b.c[1] * b.c[2] == 1) return kBlockTet;
+    } else {
+        V3<double> s[4];
+        for (int q = 0; q < 4; ++q) s[q] = mk(b.x[q], b.y[q], b.z[q]);
+        const int cls = classify_margin(s, box);
+        if (cls == CLS_NONE) return kBlockEmpty;
+        if (cls == CLS_CELL_IN_TET) return kBlockFull;
+    }
+    return work_class(b, mn, mx);
+}
+
+// set bits of m below this lane
+__device__ __forceinline__ int mbcnt64(unsigned long long m) {
+    return int(__builtin_amdgcn_mbcnt_hi(unsigned(m >> 32), __builtin_amdgcn_mbcnt_lo(unsigned(m), 0u)));
+}
+
+// Appends each lane's entry to queue `key` (none when key < 0).  Every queue holds < 64 entries before,
+// so a count reaches at most 127; an entry beyond 64 is carried.
+template <int E>
+__device__ __forceinline__ void push_blocks(BlockLds<E>& L, int lane, int key, int2 entry) {
+    int ckey = -1;
+    if (key >= 0) {
+        const int pos = atomicAdd(&L.qn[key], 1);
+        if (pos < kWaveTile) {
+            L.q[key][pos] = entry;
+        } else {
+            ckey = key;
+            L.carry[lane] = entry;
+        }
+    }
+    L.carry_key[lane] = (signed char)ckey;
+    wave_sync();
+}
+
+// This lane's column of shares.
+struct LaneShares {
+    double* a;
+    __device__ __forceinline__ void add(int i, double v) {
+        __hip_atomic_fetch_add(a + i * kWaveTile, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+    }
+};
+
+// Clips one queued block and deposits its cells, except those whose share is small against the
+// rounding of the differences: returns their mask (bit = index of the cell in the block).
+// Loader: block(entry) the block, place(entry, lo) the place of a cell of it in its grid (looked up again
+// after the clip, which needs the registers), add(entry, offset, share) the deposit.
+template <class Loader>
+__device__ __forceinline__ unsigned clip_block(const Loader& ld, int2 e, const Block& b, double* acc) {
+    const int n = b.c[0] * b.c[1] * b.c[2];
+    for (int i = 0; i < n; ++i) acc[i * kWaveTile] = 0.0;
+    LaneShares sum{acc};
+    block_shares(b.x, b.y, b.z, b.c[0], b.c[1], b.c[2], sum);
+    unsigned redo = 0u;
+    for_cells(b.c, ld.place(e, b.lo), [&](int i, int64_t at) {
+        const double f = acc[i * kWaveTile];
+        if (f >= kSmallShare) ld.add(e, at, f);
+        else if (fabs(f) >= kNoShare) redo |= 1u << i;
+    });
+    return redo;
+}
+
+// Recomputes one cell of a block alone (the paths first, first + stride, ... of exact_cell_share).  keep:
+// this lane's LDS column.
+template <class Loader>
+__device__ __forceinline__ void clip_cell(const Loader& ld, int2 e, Block b, int cell, int first, int stride, double* keep) {
+    const int q = int(udiv_small(unsigned(cell), unsigned(b.c[2]))), k = cell - q * b.c[2];
+    const int a = int(udiv_small(unsigned(q), unsigned(b.c[1]))), j = q - a * b.c[1];
+    for (int i = 0; i < 4; ++i) {
+        b.x[i] -= double(a);
+        b.y[i] -= double(j);
+        b.z[i] -= double(k);
+    }
+    b.lo[0] += a;
+    b.lo[1] += j;
+    b.lo[2] += k;
+    const double f = exact_cell_share(b.x, b.y, b.z, [&](int i) -> double& { return keep[i * kWaveTile]; }, first, stride);
+    if (f > 0.0) ld.add(e, ld.place(e, b.lo).corner, f);
+}
+
+// A wavefront's state between calls of run_wave.
+struct WaveState {
+    unsigned pend = 0u;  // cells of this lane's last block left to the exact queue
+    int2 pe = make_int2(0, 0);
+    unsigned n_exact = 0, n_partial = 0;  // this lane's recomputes, the wave's clipped blocks
+};
+
+template <int E>
+__device__ __forceinline__ void init_wave(BlockLds<E>& L, int lane) {
+    if (lane < 16) L.qn[lane] = 0;
+    L.carry_key[lane] = -1;
+    wave_sync();
+}
+
+// Feeds and clips until feed(L, lane) returns false (it appends at most one entry per lane), then, with
+// `drain`, until the queues are empty: passes filled across the classes, a full queue or the exact one
+// first.  Without `drain` every queue is left below 64 entries and nothing is carried.  A pass takes at
+// least one entry and exact passes add none, so the loop ends.
+template <int E, class Feed, class Loader>
+__device__ __forceinline__ void run_wave(BlockLds<E>& L, int lane, WaveState& w, Feed& feed, const Loader& ld, bool drain) {
+    bool draining = false;
+    for (;;) {
+        // pending cells go to the exact queue, one per lane and round, up to its 64 entries; a full exact
+        // queue is clipped first
+        const unsigned long long pm = __ballot(w.pend != 0u);
+        const int nexact = pm ? __builtin_amdgcn_readfirstlane(L.qn[kExact]) : kWaveTile;
+        if (nexact < kWaveTile) {
+            const int room = kWaveTile - nexact;
+            const int rank = mbcnt64(pm);
+            if (w.pend && rank < room) {
+                L.q[kExact][nexact + rank] = w.pe;
+                L.cell[nexact + rank] = (unsigned char)__builtin_ctz(w.pend);
+                w.pend &= w.pend - 1u;
+                ++w.n_exact;
+            }
+            wave_sync();
+            if (lane == 0) L.qn[kExact] = nexact + min(int(__popcll(pm)), room);
+            wave_sync();
+            continue;
+        }
+        // a queue to clip: full while there is work to feed, any non-empty one when draining
+        const int qv = lane < kQueues ? L.qn[lane] : 0;
+        const unsigned long long ready = __ballot(qv >= (draining ? 1 : kWaveTile));
+        if (ready) {
+            const int b = (ready >> kExact) & 1ull ? kExact : __builtin_ctzll(ready);
+            const int cnt = __builtin_amdgcn_readfirstlane(__shfl(qv, b, 64));
+            int2 e = make_int2(0, 0);
+            int cell = 0, first = 0, stride = 1;
+            bool have = false;
+            if (draining && b != kExact && cnt < kWaveTile) {
+                // up to 64 entries across all classes, from the top of each queue, lowest class first
+                const int qc = lane < kClasses ? qv : 0;
+                int pre = qc;
+                for (int d = 1; d < 8; d <<= 1) {
+                    const int o = __shfl_up(pre, d, 64);
+                    if (lane >= d) pre += o;
+                }
+                const int excl = pre - qc;
+                const int tq = lane < kClasses ? max(0, min(qc, kWaveTile - excl)) : 0;
+                for (int qi = 0; qi < kClasses; ++qi) {
+                    const int ex = __shfl(excl, qi, 64), tk = __shfl(tq, qi, 64), cq = __shfl(qc, qi, 64);
+                    if (lane >= ex && lane < ex + tk) {
+                        e = L.q[qi][cq - tk + (lane - ex)];
+                        have = true;
+                    }
+                }
+                wave_sync();
+                if (lane < kClasses) L.qn[lane] = qc - tq;
+            } else {
+                // what the count holds beyond 64 are carried entries, which take the freed positions
+                const int take = min(cnt, kWaveTile), rest = cnt - take;
+                int at = lane;
+                if (b == kExact && take <= kWaveTile / 4) {
+                    // few cells (a drain): the lanes share each one's paths, or the wave would wait for the
+                    // one with the most (196 608 tets on 64^3 cells: 424 us against 460)
+                    const int bits = 31 - __builtin_clz(unsigned(kWaveTile / take));
+                    const int shift = min(bits, 5);
+                    stride = 1 << shift;
+                    first = lane & (stride - 1);
+                    at = lane >> shift;
+                }
+                if (at < take) {
+                    e = L.q[b][at];
+                    cell = L.cell[at];
+                    have = true;
+                }
+                wave_sync();
+                if (lane == 0) L.qn[b] = rest;
+                if (rest > 0) {
+                    const bool mine = L.carry_key[lane] == b;
+                    const unsigned long long m = __ballot(mine);
+                    if (mine) {
+                        L.q[b][mbcnt64(m)] = L.carry[lane];
+                        L.carry_key[lane] = -1;
+                    }
+                }
+            }
+            wave_sync();
+            if (have) {
+                const Block blk = ld.block(e);
+                if (b == kExact) {
+                    clip_cell(ld, e, blk, cell, first, stride, &L.acc[0][lane]);
+                } else {
+                    w.pend = clip_block(ld, e, blk, &L.acc[0][lane]);
+                    w.pe = e;
+                }
+            }
+            wave_sync();
+            continue;
+        }
+        if (draining) break;
+        if (!feed(L, lane)) {
+            if (!drain) break;
+            draining = true;
+        }
+    }
+}
+
+// Tile of 64 consecutive units over items of `cnt` units each (this lane's item: [start, start + cnt)):
+// the item of unit `cursor + lane`, or -1 beyond the last.
+template <int E>
+__device__ __forceinline__ int item_of_unit(BlockLds<E>& L, int lane, unsigned start, unsigned cnt, unsigned cursor) {
+    L.mark[lane] = -1;
+    wave_sync();
+    if (cnt > 0 && start < cursor + kWaveTile && start + cnt > cursor) L.mark[int(max(start, cursor) - cursor)] = lane;
+    wave_sync();
+    int item = L.mark[lane];
+    for (int d = 1; d < 64; d <<= 1) {
+        const int o = __shfl_up(item, d, 64);
+        if (lane >= d) item = max(item, o);
+    }
+    wave_sync();
+    return item;
+}
+
+}  // namespace adeco

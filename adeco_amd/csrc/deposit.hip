@@ -200,6 +200,10 @@ hipError_t launch_add_f64_to_f32(const double* d_src, float* d_dst, int64_t n, h
     return hipGetLastError();
 }
 
+hipError_t launch_clear_grid(double* d_grid, int64_t n, hipStream_t stream) {
+    return launch_fill_f64(d_grid, n + int64_t(kCountersBytes / sizeof(double)), 0.0, stream);
+}
+
 hipError_t launch_fill_f64(double* d, int64_t n, double v, hipStream_t stream) {
     if (n <= 0) return hipSuccess;
     const unsigned nb = unsigned(n / 256 + 1 < 4096 ? n / 256 + 1 : 4096);

@@ -82,6 +82,26 @@ hipError_t launch_deposit_soup_plain(const float* d_tets, int64_t n_tets, const 
                                      double tet_mass, double* d_grid, unsigned long long* d_stats,
                                      hipStream_t stream);
 
+// ---- direct.hip: the same deposits shared by the lanes of a wave (block_wave.hpp) ----
+// Work counter and counts of one launch; zero before it.
+struct DirectCounters {
+    unsigned next, pad_;
+    unsigned long long recomputes, partials, units;
+};
+// Whether the direct deposit takes this grid and number of tets (unit scaled cells, dims < 1024).
+bool direct_deposit_fits(const GridGeom& g, int64_t n_tets);
+hipError_t launch_direct_patches(const float* d_positions, int64_t num_patches, int m, int decomp, const GridGeom& g,
+                                 double tet_mass, double* d_grid, DirectCounters* ctr, int device, hipStream_t stream);
+hipError_t launch_direct_lattice(const LatticeView& lat, int decomp, const int32_t* d_tet_ids, int64_t n_tets, const GridGeom& g,
+                                 double tet_mass, double* d_grid, DirectCounters* ctr, int device, hipStream_t stream);
+hipError_t launch_direct_soup(const float* d_tets, int64_t n_tets, const GridGeom& g, double tet_mass, double* d_grid,
+                              DirectCounters* ctr, int device, hipStream_t stream);
+// Clears a grid of n cells and the counters that follow it in the same allocation.
+constexpr size_t kCountersBytes = 64;
+static_assert(sizeof(DirectCounters) <= kCountersBytes, "counters after a grid");
+inline DirectCounters* counters_after(double* d_grid, int64_t n) { return reinterpret_cast<DirectCounters*>(d_grid + n); }
+hipError_t launch_clear_grid(double* d_grid, int64_t n, hipStream_t stream);
+
 hipError_t launch_add_f64_to_f32(const double* d_src, float* d_dst, int64_t n, hipStream_t stream);
 hipError_t launch_fill_f64(double* d, int64_t n, double v, hipStream_t stream);
 

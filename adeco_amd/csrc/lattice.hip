@@ -326,20 +326,27 @@ adeco_status adeco_lattice_deposit_grid(adeco_lattice L, int decomposition, doub
     hipError_t e = hipSetDevice(L->device);
     if (e != hipSuccess) return hip_fail(e, "hipSetDevice");
     const size_t ncell = size_t(dims) * dims * dims;
-    adeco_status st = ds.grid.reserve(ncell * sizeof(double));
+    adeco_status st = ds.grid.reserve(ncell * sizeof(double) + kCountersBytes);
     if (st) return st;
     if (tet_ids && (st = ds.pos.reserve(size_t(n_tets) * sizeof(int32_t) + 4))) return st;
     if ((st = ds.stats.reserve(kNumStats * sizeof(unsigned long long)))) return st;
     const GridGeom g = make_grid_geom(bbox6, dims, cell_scaling());
-    e = launch_fill_f64(ds.grid.as<double>(), int64_t(ncell), 0.0, ds.stream);
+    double* d_grid = ds.grid.as<double>();
+    e = launch_clear_grid(d_grid, int64_t(ncell), ds.stream);
     if (e == hipSuccess && tet_ids)
         e = hipMemcpyAsync(ds.pos.ptr, tet_ids, size_t(n_tets) * sizeof(int32_t), hipMemcpyHostToDevice, ds.stream);
     if (e == hipSuccess && stats) e = hipMemsetAsync(ds.stats.ptr, 0, kNumStats * sizeof(unsigned long long), ds.stream);
     if (e != hipSuccess) return hip_fail(e, "deposit setup");
     LatticeView lv{L->d_x, L->d_y, L->d_z, {L->np[0], L->np[1], L->np[2]}};
     if ((st = timed_begin(ds))) return st;
-    e = launch_deposit_lattice_plain(lv, decomposition, tet_ids ? ds.pos.as<int32_t>() : nullptr, n_tets, g, tet_mass,
-                                     ds.grid.as<double>(), stats ? ds.stats.as<unsigned long long>() : nullptr, ds.stream);
+    // (work statistics count the one-tet-per-thread kernel's steps)
+    const int32_t* d_ids = tet_ids ? ds.pos.as<int32_t>() : nullptr;
+    if (!stats && direct_deposit_fits(g, n_tets))
+        e = launch_direct_lattice(lv, decomposition, d_ids, n_tets, g, tet_mass, d_grid, counters_after(d_grid, int64_t(ncell)),
+                                  L->device, ds.stream);
+    else
+        e = launch_deposit_lattice_plain(lv, decomposition, d_ids, n_tets, g, tet_mass, d_grid,
+                                         stats ? ds.stats.as<unsigned long long>() : nullptr, ds.stream);
     if (e != hipSuccess) return hip_fail(e, "deposit launch");
     if ((st = timed_end(ds))) return st;
     e = hipMemcpyAsync(grid_out, ds.grid.ptr, ncell * sizeof(double), hipMemcpyDeviceToHost, ds.stream);
@@ -367,11 +374,12 @@ adeco_status adeco_deposit_soup(int device_id, const float* tets, int64_t n_tets
     hipError_t e = hipSetDevice(device_id);
     if (e != hipSuccess) return hip_fail(e, "hipSetDevice");
     const size_t ncell = size_t(dims) * dims * dims;
-    if ((st = ds.grid.reserve(ncell * sizeof(double)))) return st;
+    if ((st = ds.grid.reserve(ncell * sizeof(double) + kCountersBytes))) return st;
     if ((st = ds.pos.reserve(size_t(n_tets) * 12 * sizeof(float) + 4))) return st;
     if ((st = ds.stats.reserve(kNumStats * sizeof(unsigned long long)))) return st;
     const GridGeom g = make_grid_geom(bbox6, dims, cell_scaling());
-    e = launch_fill_f64(ds.grid.as<double>(), int64_t(ncell), 0.0, ds.stream);
+    double* d_grid = ds.grid.as<double>();
+    e = launch_clear_grid(d_grid, int64_t(ncell), ds.stream);
     if (e == hipSuccess) e = hipMemcpyAsync(ds.pos.ptr, tets, size_t(n_tets) * 12 * sizeof(float), hipMemcpyHostToDevice, ds.stream);
     if (e == hipSuccess && stats) e = hipMemsetAsync(ds.stats.ptr, 0, kNumStats * sizeof(unsigned long long), ds.stream);
     if (e != hipSuccess) return hip_fail(e, "soup setup");
@@ -379,8 +387,12 @@ adeco_status adeco_deposit_soup(int device_id, const float* tets, int64_t n_tets
     if (mode == ADECO_MODE_BATCHED) {
         if ((st = deposit_soup_batched(ds, ds.pos.as<float>(), n_tets, g, tet_mass, precision, ds.grid.as<double>()))) return st;
     } else {
-        e = launch_deposit_soup_plain(ds.pos.as<float>(), n_tets, g, tet_mass, ds.grid.as<double>(),
-                                      stats ? ds.stats.as<unsigned long long>() : nullptr, ds.stream);
+        if (!stats && direct_deposit_fits(g, n_tets))
+            e = launch_direct_soup(ds.pos.as<float>(), n_tets, g, tet_mass, d_grid, counters_after(d_grid, int64_t(ncell)), device_id,
+                                   ds.stream);
+        else
+            e = launch_deposit_soup_plain(ds.pos.as<float>(), n_tets, g, tet_mass, d_grid,
+                                          stats ? ds.stats.as<unsigned long long>() : nullptr, ds.stream);
         if (e != hipSuccess) return hip_fail(e, "soup launch");
     }
     if ((st = timed_end(ds))) return st;

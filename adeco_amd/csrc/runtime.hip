@@ -178,13 +178,15 @@ adeco_status deposit_patches_on_device(int dev, size_t first_patch, size_t n_pat
     const size_t patches_per_pass = std::max<size_t>(1, std::min(n_patches, avail / per_patch));
     if (patches_per_pass * per_patch > avail)
         return fail(ADECO_EOVERFLOW, "memory budget too small for one meta-patch");
-    if ((st = ds.grid.reserve(grid_bytes))) return st;
+    if ((st = ds.grid.reserve(grid_bytes + kCountersBytes))) return st;
     if ((st = ds.pos.reserve(patches_per_pass * patch_bytes))) return st;
     DevBuf& soup = ds.soup;
     if (batched && (st = soup.reserve(patches_per_pass * soup_bytes))) return st;
     const GridGeom g = make_grid_geom(bbox, dims, cell_scaling());
-    if ((e = launch_fill_f64(ds.grid.as<double>(), int64_t(ncell), 0.0, ds.stream)) != hipSuccess)
-        return hip_fail(e, "grid clear");
+    double* d_grid = ds.grid.as<double>();
+    DirectCounters* ctr = counters_after(d_grid, int64_t(ncell));
+    const bool direct = direct_deposit_fits(g, int64_t(patches_per_pass * tets_per_patch));
+    if ((e = launch_clear_grid(d_grid, int64_t(ncell), ds.stream)) != hipSuccess) return hip_fail(e, "grid clear");
     double total_ms = 0.0;
     for (size_t done = 0; done < n_patches; done += patches_per_pass) {
         const size_t np = std::min(patches_per_pass, n_patches - done);
@@ -201,8 +203,13 @@ adeco_status deposit_patches_on_device(int dev, size_t first_patch, size_t n_pat
             continue;
         }
         if ((st = timed_begin(ds))) return st;
-        e = launch_deposit_patches_plain(ds.pos.as<float>(), int64_t(np), m, decomp, g, tet_mass, ds.grid.as<double>(),
-                                         nullptr, ds.stream);
+        // the tets of a pass shared by the lanes of each wave; one per thread where the cells are not unit
+        // cells (the reference's scaling) or the grid is beyond the block form
+        if (direct && done) e = launch_zero_u32(&ctr->next, 1, ds.stream);
+        if (e == hipSuccess)
+            e = direct ? launch_direct_patches(ds.pos.as<float>(), int64_t(np), m, decomp, g, tet_mass, d_grid, ctr, dev, ds.stream)
+                       : launch_deposit_patches_plain(ds.pos.as<float>(), int64_t(np), m, decomp, g, tet_mass, d_grid, nullptr,
+                                                      ds.stream);
         if (e != hipSuccess) return hip_fail(e, "deposit launch");
         if ((st = timed_end(ds))) return st;
         total_ms += g_last_kernel_ms;

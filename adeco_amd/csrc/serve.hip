@@ -828,14 +828,18 @@ adeco_status adeco_roi_deposit_plain(adeco_lattice L, int decomposition, double 
     int64_t n = 0;
     if ((st = sel.select(ds.stream, lv, ct, rf, ds.pos, n, [](size_t) { return true; }))) return st;
     const int64_t cells = int64_t(dims) * dims * dims;
-    if ((st = ds.grid.reserve(size_t(cells) * 8)) || (st = ds.scratch.reserve(size_t(cells) * 4))) return st;
+    if ((st = ds.grid.reserve(size_t(cells) * 8 + kCountersBytes)) || (st = ds.scratch.reserve(size_t(cells) * 4))) return st;
     const GridGeom g = roi_geom(roi6, dims);
-    e = launch_fill_f64(ds.grid.as<double>(), cells, 0.0, ds.stream);
+    double* d_grid = ds.grid.as<double>();
+    e = launch_clear_grid(d_grid, cells, ds.stream);
     if (e != hipSuccess) return hip_fail(e, "roi_deposit_plain()");
     if ((st = timed_begin(ds))) return st;
     if (n > 0) {
-        e = launch_deposit_lattice_plain(lv, decomposition, ds.pos.as<int32_t>(), n, g, tet_mass, ds.grid.as<double>(), nullptr,
-                                         ds.stream);
+        if (direct_deposit_fits(g, n))
+            e = launch_direct_lattice(lv, decomposition, ds.pos.as<int32_t>(), n, g, tet_mass, d_grid, counters_after(d_grid, cells),
+                                      L->device, ds.stream);
+        else
+            e = launch_deposit_lattice_plain(lv, decomposition, ds.pos.as<int32_t>(), n, g, tet_mass, d_grid, nullptr, ds.stream);
         if (e != hipSuccess) return hip_fail(e, "roi_deposit_plain() launch");
     }
     if ((st = timed_end(ds))) return st;

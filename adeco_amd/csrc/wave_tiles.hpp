@@ -45,6 +45,12 @@ __device__ __forceinline__ int64_t shfl_i64(int64_t v, int src) {
     return int64_t((uint64_t(unsigned(hi)) << 32) | unsigned(lo));
 }
 
+__device__ __forceinline__ int64_t shfl_up_i64(int64_t v, int d) {
+    const int lo = __shfl_up(int(uint64_t(v) & 0xffffffffu), d, 64);
+    const int hi = __shfl_up(int(uint64_t(v) >> 32), d, 64);
+    return int64_t((uint64_t(unsigned(hi)) << 32) | unsigned(lo));
+}
+
 // What a tile's classification needs first: its source slot and index, its first pair, the number
 // of pairs it touches and, per lane, the candidate offset of pair p0 + lane.  Loaded one tile
 // ahead, so that these dependent loads overlap the previous tile's work.

@@ -228,12 +228,21 @@ adeco_status deposit_leaves_plain(adeco_octree_s* T, int dims, int decomposition
     const int64_t cells = int64_t(dims) * dims * dims;
     const LatticeView lv{L->d_x, L->d_y, L->d_z, {L->np[0], L->np[1], L->np[2]}};
     const int scaling = cell_scaling();
+    // one launch per leaf, each with a work counter of its own
+    adeco_status st = T->d_counters.reserve(size_t(nl) * sizeof(DirectCounters));
+    if (st) return st;
+    DirectCounters* ctr = T->d_counters.as<DirectCounters>();
+    hipError_t ez = launch_zero_u32(reinterpret_cast<unsigned*>(ctr), int(nl * int64_t(sizeof(DirectCounters) / 4)), ds.stream);
+    if (ez != hipSuccess) return hip_fail(ez, "leaf deposit counters");
     for (int64_t l = 0; l < nl; ++l) {
         const int64_t b = T->leaf_tet_offset[l], n = T->leaf_tet_offset[l + 1] - b;
         if (!n) continue;
         const GridGeom g = T->leaf_geom(int(l), dims, scaling);
-        hipError_t e = launch_deposit_lattice_plain(lv, decomposition, T->d_pairs.as<int32_t>() + b, n, g, tet_mass,
-                                                    T->d_grids.as<double>() + l * cells, nullptr, ds.stream);
+        const int32_t* ids = T->d_pairs.as<int32_t>() + b;
+        double* grid = T->d_grids.as<double>() + l * cells;
+        const hipError_t e = direct_deposit_fits(g, n)
+                                 ? launch_direct_lattice(lv, decomposition, ids, n, g, tet_mass, grid, ctr + l, L->device, ds.stream)
+                                 : launch_deposit_lattice_plain(lv, decomposition, ids, n, g, tet_mass, grid, nullptr, ds.stream);
         if (e != hipSuccess) return hip_fail(e, "leaf deposit launch");
     }
     return ADECO_OK;
