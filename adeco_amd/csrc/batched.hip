@@ -862,6 +862,11 @@ hipError_t launch_scan_u32(const unsigned* in, int64_t n, int64_t* out, int64_t*
     return hipGetLastError();
 }
 
+hipError_t launch_pair_grid(hipStream_t stream, const int64_t* grid_off, int n_grids, int64_t cap, int32_t* pair_grid) {
+    hipLaunchKernelGGL(k_pair_grid, dim3(unsigned(n_grids)), dim3(256), 0, stream, grid_off, cap, pair_grid);
+    return hipGetLastError();
+}
+
 // Lays out the slab of a candidate space for up to n_pairs pairs and enqueues pair setup and the
 // candidate scan; n_dev (nullable) is the pair count on the device, capped at n_pairs.
 static void enqueue_candidate_space(hipStream_t stream, const LatticeView& lat, const PackedCorners& ct,
@@ -886,8 +891,7 @@ static void enqueue_candidate_space(hipStream_t stream, const LatticeView& lat, 
     cs.n_cand = 0;
     cs.n_tiles = 0;
     if (n_pairs == 0) return;
-    if (pair_grid)
-        hipLaunchKernelGGL(k_pair_grid, dim3(unsigned(n_grids)), dim3(256), 0, stream, grid_off, n_pairs, pair_grid);
+    if (pair_grid) (void)launch_pair_grid(stream, grid_off, n_grids, n_pairs, pair_grid);
     if (form == kFormBlocks)
         (void)launch_block_setup(stream, lat, ct, pairs, n_pairs, n_dev, grid_off, n_grids, pair_grid, d_grids, tet_mass,
                                  cs.cand, cs.pd);
@@ -1024,10 +1028,58 @@ adeco_status prepare_leaves_batched(adeco_octree_s* T, hipStream_t stream, int d
     return ADECO_OK;
 }
 
-// Leaf deposit of an octree: one candidate space over all leaves, one persistent launch.
+adeco_status deposit_leaves_direct(adeco_octree_s* T, int dims, int decomposition, double tet_mass, bool only_small, bool& taken) {
+    adeco_lattice_s* L = T->L;
+    DeviceState& ds = *L->ds;
+    taken = false;
+    const int nl = int(T->leaves_dfs.size());
+    const int64_t P = T->leaf_tet_offset[nl];
+    const int64_t cells = int64_t(dims) * dims * dims;
+    // tets of few blocks: a pair line (128 bytes written once and read twice, a scan, a tile map) costs more than
+    // reading the tet again; beyond about 1.5 blocks per pair, which 4 pairs per cell stand for, the blocks of
+    // a pair share its line.  512 leaves, 15.3 M pairs, ms direct | with lines: 16^3 cells (7.3 per cell) 4.26 |
+    // 4.66, 20^3 (3.7) 5.95 | 5.96, 24^3 (2.2) 8.8 | 8.1, 32^3 (0.9) 17.6 | 15.7.
+    const bool small = P >= 4 * nl * cells;
+    if (only_small && !small) return ADECO_OK;
+    std::vector<GridDesc>& gd = T->leaf_desc;  // (alive until the upload has been read)
+    gd.resize(nl);
+    const int scaling = cell_scaling();
+    for (int l = 0; l < nl; ++l) gd[l] = make_grid_desc(T->leaf_geom(l, dims, scaling), (long long)(l * cells));
+    if (!direct_deposit_fits(gd.data(), nl, P)) return ADECO_OK;
+    taken = true;
+    T->d_fallback = nullptr;
+    if (P == 0) return ADECO_OK;
+    adeco_status st;
+    if ((st = T->d_work.reserve(size_t(P) * sizeof(int32_t))) || (st = T->d_leaf_geom.reserve(gd.size() * sizeof(GridDesc))) ||
+        (st = T->d_counters.reserve(kCountersBytes)))
+        return st;
+    int32_t* pair_grid = T->d_work.as<int32_t>();
+    DirectCounters* ctr = T->d_counters.as<DirectCounters>();
+    const LatticeView lv{L->d_x, L->d_y, L->d_z, {L->np[0], L->np[1], L->np[2]}};
+    hipError_t e = hipMemcpyAsync(T->d_leaf_geom.ptr, gd.data(), gd.size() * sizeof(GridDesc), hipMemcpyHostToDevice, ds.stream);
+    if (e == hipSuccess) e = launch_pair_grid(ds.stream, T->d_leaf_offset.as<int64_t>(), nl, P, pair_grid);
+    if (e == hipSuccess) e = launch_zero_u32(reinterpret_cast<unsigned*>(ctr), int(sizeof(DirectCounters) / 4), ds.stream);
+    if (e == hipSuccess) e = hipEventRecord(ds.evk0, ds.stream);
+    if (e == hipSuccess)
+        e = launch_direct_leaves(lv, decomposition, T->d_pairs.as<int32_t>(), pair_grid, P, T->d_leaf_geom.as<GridDesc>(), dims, small, tet_mass,
+                                 T->d_grids.as<double>(), ctr, L->device, ds.stream);
+    if (e == hipSuccess) e = hipEventRecord(ds.evk1, ds.stream);
+    if (e != hipSuccess) return hip_fail(e, "leaf deposit launch");
+    T->last_candidates = -1;  // counted by the kernel
+    T->d_fallback = &ctr->recomputes;
+    return ADECO_OK;
+}
+
+// Leaf deposit of an octree in one persistent launch: straight from its pairs (FP64 on unit cells), or one
+// candidate space over all leaves.
 adeco_status deposit_leaves_batched(adeco_octree_s* T, int dims, int decomposition, double tet_mass, int precision) {
     adeco_lattice_s* L = T->L;
     DeviceState& ds = *L->ds;
+    if (precision == ADECO_PREC_FP64 && dims <= 1023) {
+        bool taken = false;
+        const adeco_status s = deposit_leaves_direct(T, dims, decomposition, tet_mass, true, taken);
+        if (s || taken) return s;
+    }
     TileSource src;
     adeco_status st = prepare_leaves_batched(T, ds.stream, dims, decomposition, tet_mass, precision, T->d_leaf_geom, T->d_work,
                                              T->d_tiles, T->d_grids.as<double>(), src);

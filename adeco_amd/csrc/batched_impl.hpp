@@ -141,6 +141,18 @@ adeco_status prepare_leaves_batched(adeco_octree_s* T, hipStream_t stream, int d
                                     int precision, DevBuf& geom, DevBuf& work, DevBuf& tiles, double* grids,
                                     TileSource& src);
 
+// grid index of every pair of n_grids grid-major pairs (below cap)
+hipError_t launch_pair_grid(hipStream_t stream, const int64_t* grid_off, int n_grids, int64_t cap, int32_t* pair_grid);
+
+// The direct form over the (leaf, tet) pairs of an octree (direct.hip).
+bool direct_deposit_fits(const GridDesc* grids, int64_t n, int64_t n_tets);
+hipError_t launch_direct_leaves(const LatticeView& lat, int decomp, const int32_t* d_pairs, const int32_t* d_pair_grid,
+                                int64_t n_pairs, const GridDesc* d_grids, int dims, bool small_tets, double tet_mass,
+                                double* d_grid_buf, DirectCounters* ctr, int device, hipStream_t stream);
+// Leaf deposit in that form, all leaves in one launch; taken = false (and nothing done) where it does not fit, or
+// where pair lines are faster and wanted (`only_small`).
+adeco_status deposit_leaves_direct(adeco_octree_s* T, int dims, int decomposition, double tet_mass, bool only_small, bool& taken);
+
 // The block form's kernels (blocks.hip).
 hipError_t launch_block_setup(hipStream_t stream, const LatticeView& lat, const PackedCorners& ct, const int32_t* pairs,
                               int64_t n_pairs, const int64_t* n_dev, const int64_t* grid_off, int n_grids,

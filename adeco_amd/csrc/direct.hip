@@ -1,5 +1,6 @@
-// Direct block deposit: tets straight from their vertices onto one grid in a single launch, with no pair
-// lines, scan or tile map in between (the plain form of the FP64 deposit on grids of unit scaled cells).
+// Direct block deposit: tets straight from their vertices onto their grids in a single launch, with no pair
+// lines, scan or tile map in between (the FP64 deposit on grids of unit scaled cells: the plain forms, and
+// the leaf deposit where most pairs are a block or two).
 //
 // A wavefront takes `per_item` consecutive tets from a work counter, one per lane: covered range and
 // number of blocks (block_wave.hpp).  The blocks of the item are then walked 64 at a time, one per lane;
@@ -7,10 +8,11 @@
 // and full queues are clipped by the whole wave.  So a wave's lanes share the cells of a large tet, and
 // nothing but the tets is read from memory.
 // Against the one-tet-per-thread kernel (deposit.hip), whose waves run as long as their largest tet
-// walks its cells: one meta-patch of 2 058 tets on 16^3 cells 110 us against 900-1130, a leaf's 98 784 tets
-// on 16^3 cells 205 against 1420-1530, 196 608 tets on 64^3 cells 0.42 ms against 3.8.  What bounds it: a
-// small launch lasts as long as one wave's chain of passes (classify, clip, recompute: 20-30 us each, at
-// mostly one wave per SIMD); a large one is bound as the batched form is (blocks.hip).
+// walks its cells: one meta-patch of 2 058 tets on 16^3 cells 120 us against 900-1130, a leaf's 98 784 tets
+// on 16^3 cells 215 against 1420-1530, 196 608 tets on 64^3 cells 0.43 ms against 3.8.  All leaves of an
+// octree in one launch instead of one each: 64 leaves, 1.86 M pairs, 16^3 cells 0.77 ms against 15.2.
+// What bounds it: a small launch lasts as long as one wave's chain of passes (classify, clip, recompute:
+// 20-30 us each, at mostly one wave per SIMD); a large one is bound as the batched form is (blocks.hip).
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -33,8 +35,14 @@ constexpr int kCells = 16;
 using Lds = BlockLds<kCells>;
 static_assert((sizeof(Lds) * kWaves + 1279) / 1280 * 1280 * 3 <= 160 * 1024, "3 workgroups per CU");
 
+// Tets of one grid.
+struct OneGrid {
+    GridDesc g;
+    __device__ __forceinline__ const GridDesc& grid(int) const { return g; }
+};
+
 // The tets of a lattice: all of them, or those listed.
-struct LatticeTets {
+struct LatticeTets : OneGrid {
     LatticeView lat;
     PackedCorners ct;
     const int32_t* ids;
@@ -44,8 +52,22 @@ struct LatticeTets {
     }
 };
 
+// The (leaf, tet) pairs of an octree, each with the grid of its leaf.
+struct LeafTets {
+    LatticeView lat;
+    PackedCorners ct;
+    const int32_t* pairs;
+    const int32_t* pair_grid;
+    const GridDesc* grids;
+    __device__ __forceinline__ const GridDesc& grid(int i) const { return grids[pair_grid[i]]; }
+    __device__ __forceinline__ bool fetch(int64_t i, V3<double> v[4]) const {
+        lattice_tet_vertices(lat, ct, pairs[i], v);
+        return true;
+    }
+};
+
 // A tet soup: 4 vertices of 3 floats each.
-struct SoupTets {
+struct SoupTets : OneGrid {
     const float* p;
     __device__ __forceinline__ bool fetch(int64_t i, V3<double> v[4]) const {
         const float* t = p + 12 * i;
@@ -56,7 +78,7 @@ struct SoupTets {
 
 // The 6 tets of every cell of meta-patches of m^3 cells (AoS positions); a cell with a 666 sentinel
 // vertex has none (AdDepositTets2Grid.h:1029-1038).
-struct PatchTets {
+struct PatchTets : OneGrid {
     const float* pos;
     int m;
     PackedCorners pc;
@@ -112,16 +134,20 @@ __device__ __forceinline__ TetCover cover_of(const V3<double> v[4], const GridDe
 template <class Tets>
 struct DirectLoader {
     const Tets& tets;
-    const GridDesc& g;
     double* grid;
     double tet_mass;
     __device__ __forceinline__ Block block(int2 e) const {
         V3<double> v[4];
         (void)tets.fetch(e.x, v);
-        const TetCover t = cover_of(v, g);
+        const TetCover t = cover_of(v, tets.grid(e.x));
         return make_block<kCells>(t.lo, t.e, t.s, unsigned(e.y) & kUnits);
     }
-    __device__ __forceinline__ Place place(int2 e, const int lo[3]) const { return place_of(lo, int(unsigned(e.y) >> 29), g.dims); }
+    __device__ __forceinline__ Place place(int2 e, const int lo[3]) const {
+        const GridDesc& g = tets.grid(e.x);
+        Place p = place_of(lo, int(unsigned(e.y) >> 29), g.dims);
+        p.corner += g.base;
+        return p;
+    }
     __device__ __forceinline__ void add(int2, int64_t at, double share) const { unsafeAtomicAdd(grid + at, tet_mass * share); }
     static constexpr unsigned kUnits = (1u << 29) - 1u;  // below the axis order's 3 bits
 };
@@ -129,37 +155,42 @@ struct DirectLoader {
 template <class Tets>
 struct DirectFeed {
     const Tets& tets;
-    const GridDesc& g;
     double* grid;
     double tet_mass;
-    int64_t n_tets;
-    int per_item;
+    unsigned n_tets, per_item, per_pop;
     unsigned* counter;
     WaveState& w;
     int64_t n_units = 0;
-    // the current item: its first tet, this lane's blocks [start, start + cnt), their total, and the next
-    // block to walk
-    int64_t first = 0;
+    // the tets taken from the counter and not yet begun; the current item: its first tet, this lane's blocks
+    // [start, start + cnt), their total, and the next block to walk
+    unsigned next = 0, end = 0, first = 0;
     unsigned start = 0, cnt = 0, total = 0, cursor = 0;
 
     // One step: a new item (whose blocks follow at once when no tet has more than one), or the next 64
     // blocks of the current one.
     __device__ __forceinline__ bool operator()(Lds& L, int lane) {
         const bool fresh = cursor >= total;
-        int64_t t;  // this lane's tet, its block below
+        unsigned t;  // this lane's tet, its block below
         bool live;
         unsigned unit = 0;
         if (fresh) {
-            unsigned item = 0;
-            if (lane == 0) item = atomicAdd(counter, 1u);
-            first = int64_t(__builtin_amdgcn_readfirstlane(item)) * per_item;
-            if (first >= n_tets) return false;
-            t = first + lane;
-            live = lane < per_item && t < n_tets;
+            if (next >= end) {
+                unsigned pop = 0;
+                if (lane == 0) pop = atomicAdd(counter, 1u);
+                const int64_t at = int64_t(__builtin_amdgcn_readfirstlane(pop)) * per_pop;
+                if (at >= n_tets) return false;
+                next = unsigned(at);
+                end = unsigned(min(at + per_pop, int64_t(n_tets)));
+            }
+            first = next;
+            next += per_item;
+            t = first + unsigned(lane);
+            live = unsigned(lane) < per_item && t < end;
+            n_units += __popcll(__ballot(live));  // (a tet without volume counts as one block)
         } else {
             const int item = item_of_unit(L, lane, start, cnt, cursor);
             const unsigned item_start = unsigned(__shfl(int(start), max(item, 0), 64));
-            t = first + item;
+            t = first + unsigned(max(item, 0));
             live = cursor + unsigned(lane) < total;
             unit = cursor + unsigned(lane) - item_start;
             cursor += kWaveTile;
@@ -170,7 +201,7 @@ struct DirectFeed {
         if (live) {
             V3<double> v[4];
             live = tets.fetch(t, v);
-            c = cover_of(v, g);
+            c = cover_of(v, tets.grid(int(t)));
             code = c.code;
             vol = vol6(v[0], v[1], v[2], v[3]);
             live = live && vol != 0.0;
@@ -183,17 +214,16 @@ struct DirectFeed {
             }
             cursor = total = 0;
             if (__ballot(cnt > 1)) {
-                unsigned end = cnt;
+                unsigned last = cnt;
                 for (int d = 1; d < 64; d <<= 1) {
-                    const unsigned o = unsigned(__shfl_up(int(end), d, 64));
-                    if (lane >= d) end += o;
+                    const unsigned o = unsigned(__shfl_up(int(last), d, 64));
+                    if (lane >= d) last += o;
                 }
-                start = end - cnt;
-                total = unsigned(__builtin_amdgcn_readlane(int(end), 63));
-                n_units += total;
+                start = last - cnt;
+                total = unsigned(__builtin_amdgcn_readlane(int(last), 63));
+                n_units += int64_t(total) - __popcll(__ballot(cnt > 0));
                 return true;
             }
-            n_units += __popcll(__ballot(live));
         }
         if (live) {
             // positively oriented in the cover's axis order (the face tests need it)
@@ -206,8 +236,10 @@ struct DirectFeed {
             const Block b = make_block<kCells>(c.lo, c.e, c.s, unit);
             key = classify_block(b);
             if (key == kBlockTet || key == kBlockFull) {
+                const GridDesc& g = tets.grid(int(t));
                 const double m = key == kBlockTet ? tet_mass : tet_mass * (g.cell_vol / fabs(vol / 6.0));
-                for_cells(b.c, place_of(b.lo, code, g.dims), [&](int, int64_t at) { unsafeAtomicAdd(grid + at, m); });
+                double* to = grid + g.base;
+                for_cells(b.c, place_of(b.lo, code, g.dims), [&](int, int64_t at) { unsafeAtomicAdd(to + at, m); });
             }
         }
         push_blocks(L, lane, key, make_int2(int(t), int(unit | unsigned(code) << 29)));
@@ -217,22 +249,23 @@ struct DirectFeed {
 };
 
 template <class Tets>
-__global__ void __launch_bounds__(kThreads, 3) k_deposit_direct(Tets tets, int64_t n_tets, int per_item, GridDesc g, double tet_mass,
-                                                                double* __restrict__ grid, DirectCounters* __restrict__ ctr) {
+__global__ void __launch_bounds__(kThreads, 3) k_deposit_direct(Tets tets, unsigned n_tets, unsigned per_item, unsigned per_pop,
+                                                                double tet_mass, double* __restrict__ grid,
+                                                                DirectCounters* __restrict__ ctr) {
     __shared__ Lds lds[kWaves];
     const int lane = threadIdx.x & 63;
     Lds& L = lds[threadIdx.x >> 6];
     init_wave(L, lane);
     WaveState w;
-    DirectFeed<Tets> feed{tets, g, grid, tet_mass, n_tets, per_item, &ctr->next, w};
-    run_wave(L, lane, w, feed, DirectLoader<Tets>{tets, g, grid, tet_mass}, true);
+    DirectFeed<Tets> feed{tets, grid, tet_mass, n_tets, per_item, per_pop, &ctr->next, w};
+    run_wave(L, lane, w, feed, DirectLoader<Tets>{tets, grid, tet_mass}, true);
     if (lane == 0 && w.n_partial) atomicAdd(&ctr->partials, (unsigned long long)w.n_partial);
     if (lane == 0 && feed.n_units) atomicAdd(&ctr->units, (unsigned long long)feed.n_units);
     if (w.n_exact) atomicAdd(&ctr->recomputes, (unsigned long long)w.n_exact);
 }
 
 template <class Tets>
-hipError_t launch(const Tets& tets, int64_t n_tets, const GridDesc& g, double tet_mass, double* grid, DirectCounters* ctr,
+hipError_t launch(const Tets& tets, int64_t n_tets, int dims, bool small_tets, double tet_mass, double* grid, DirectCounters* ctr,
                   int device, hipStream_t stream) {
     if (n_tets <= 0) return hipSuccess;
     int cus = 256;
@@ -242,39 +275,54 @@ hipError_t launch(const Tets& tets, int64_t n_tets, const GridDesc& g, double te
     // per resident wave
     const int64_t waves = int64_t(cus) * 3 * kWaves;
     // (64 tets of up to 2^26 blocks each would overflow their 32-bit sum on grids beyond 512^3)
-    int per_item = g.dims <= 512 ? 64 : 32;
+    int per_item = dims <= 512 ? 64 : 32;
     while (per_item > 1 && n_tets < 2 * waves * per_item) per_item >>= 1;
     const int64_t items = (n_tets + per_item - 1) / per_item;
-    const unsigned blocks = unsigned(std::min<int64_t>((items + kWaves - 1) / kWaves, int64_t(cus) * 3));
-    hipLaunchKernelGGL(k_deposit_direct<Tets>, dim3(blocks), dim3(kThreads), 0, stream, tets, n_tets, per_item, g, tet_mass, grid,
-                       ctr);
+    const WaveLaunch w = wave_launch(items, block_occupancy(), kWaves, device);
+    // items per pop: one where the tets' blocks may differ much in number (45 M blocks of 6.7 M pairs on 32^3-cell
+    // leaves: 18.3 ms against 23.2 with 4), else up to the launch shape's with at least 8 pops per wave (15.3 M
+    // pairs on 16^3-cell leaves: 4.19 ms against 4.37 with 1)
+    const int64_t chunk = small_tets ? std::max<int64_t>(1, std::min<int64_t>(w.chunk, items / (8 * waves))) : 1;
+    hipLaunchKernelGGL(k_deposit_direct<Tets>, dim3(w.grid), dim3(kThreads), 0, stream, tets, unsigned(n_tets), unsigned(per_item),
+                       unsigned(per_item * chunk), tet_mass, grid, ctr);
     return hipGetLastError();
 }
 
 }  // namespace
 
-bool direct_deposit_fits(const GridGeom& g, int64_t n_tets) {
+bool direct_deposit_fits(const GridDesc* grids, int64_t n, int64_t n_tets) {
     // unit scaled cells (block planes are shared by neighbouring cells), block indices of 29 bits and tet
     // indices of 31
+    return deposit_form(ADECO_PREC_FP64, grids, n) == kFormBlocks && grids[0].dims <= 1023 && n_tets < (int64_t(1) << 31) - 2;
+}
+
+bool direct_deposit_fits(const GridGeom& g, int64_t n_tets) {
     const GridDesc d = make_grid_desc(g, 0);
-    return deposit_form(ADECO_PREC_FP64, &d, 1) == kFormBlocks && g.dims <= 1023 && n_tets < (int64_t(1) << 31);
+    return direct_deposit_fits(&d, 1, n_tets);
 }
 
 hipError_t launch_direct_lattice(const LatticeView& lat, int decomp, const int32_t* d_ids, int64_t n_tets, const GridGeom& g,
                                  double tet_mass, double* d_grid, DirectCounters* ctr, int device, hipStream_t stream) {
-    return launch(LatticeTets{lat, pack_corners(corner_table(decomp)), d_ids}, n_tets, make_grid_desc(g, 0), tet_mass, d_grid,
-                  ctr, device, stream);
+    return launch(LatticeTets{{make_grid_desc(g, 0)}, lat, pack_corners(corner_table(decomp)), d_ids}, n_tets, g.dims, false, tet_mass,
+                  d_grid, ctr, device, stream);
+}
+
+hipError_t launch_direct_leaves(const LatticeView& lat, int decomp, const int32_t* d_pairs, const int32_t* d_pair_grid,
+                                int64_t n_pairs, const GridDesc* d_grids, int dims, bool small_tets, double tet_mass,
+                                double* d_grid_buf, DirectCounters* ctr, int device, hipStream_t stream) {
+    return launch(LeafTets{lat, pack_corners(corner_table(decomp)), d_pairs, d_pair_grid, d_grids}, n_pairs, dims, small_tets, tet_mass,
+                  d_grid_buf, ctr, device, stream);
 }
 
 hipError_t launch_direct_soup(const float* d_tets, int64_t n_tets, const GridGeom& g, double tet_mass, double* d_grid,
                               DirectCounters* ctr, int device, hipStream_t stream) {
-    return launch(SoupTets{d_tets}, n_tets, make_grid_desc(g, 0), tet_mass, d_grid, ctr, device, stream);
+    return launch(SoupTets{{make_grid_desc(g, 0)}, d_tets}, n_tets, g.dims, false, tet_mass, d_grid, ctr, device, stream);
 }
 
 hipError_t launch_direct_patches(const float* d_pos, int64_t num_patches, int m, int decomp, const GridGeom& g, double tet_mass,
                                  double* d_grid, DirectCounters* ctr, int device, hipStream_t stream) {
-    return launch(PatchTets{d_pos, m, pack_corners(corner_table(decomp))}, num_patches * m * m * m * 6, make_grid_desc(g, 0),
-                  tet_mass, d_grid, ctr, device, stream);
+    return launch(PatchTets{{make_grid_desc(g, 0)}, d_pos, m, pack_corners(corner_table(decomp))}, num_patches * m * m * m * 6, g.dims,
+                  false, tet_mass, d_grid, ctr, device, stream);
 }
 
 }  // namespace adeco

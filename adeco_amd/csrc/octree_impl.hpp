@@ -4,6 +4,7 @@
 #include <cstdint>
 #include <vector>
 
+#include "batched_impl.hpp"
 #include "kernels.hpp"
 #include "lattice_impl.hpp"
 #include "runtime.hpp"
@@ -45,6 +46,7 @@ struct adeco_octree_s {
     // leaf grids of the last deposit (device, FP64, leaf-major in DFS leaf order)
     int grid_dims = 0;
     adeco::DevBuf d_grids, d_leaf_geom, d_work, d_tiles, d_counters;
+    std::vector<adeco::GridDesc> leaf_desc;  // the leaves' grids, as uploaded by the last direct deposit
     int64_t last_candidates = 0;            // (tet, candidate) pairs of the last batched deposit
     unsigned long long* d_fallback = nullptr;  // FP64 recomputes of the last mixed-precision deposit
 

@@ -228,21 +228,16 @@ adeco_status deposit_leaves_plain(adeco_octree_s* T, int dims, int decomposition
     const int64_t cells = int64_t(dims) * dims * dims;
     const LatticeView lv{L->d_x, L->d_y, L->d_z, {L->np[0], L->np[1], L->np[2]}};
     const int scaling = cell_scaling();
-    // one launch per leaf, each with a work counter of its own
-    adeco_status st = T->d_counters.reserve(size_t(nl) * sizeof(DirectCounters));
-    if (st) return st;
-    DirectCounters* ctr = T->d_counters.as<DirectCounters>();
-    hipError_t ez = launch_zero_u32(reinterpret_cast<unsigned*>(ctr), int(nl * int64_t(sizeof(DirectCounters) / 4)), ds.stream);
-    if (ez != hipSuccess) return hip_fail(ez, "leaf deposit counters");
+    bool taken = false;
+    const adeco_status st = deposit_leaves_direct(T, dims, decomposition, tet_mass, false, taken);
+    if (st || taken) return st;
+    // leaf by leaf, one tet per thread (the reference's scaling)
     for (int64_t l = 0; l < nl; ++l) {
         const int64_t b = T->leaf_tet_offset[l], n = T->leaf_tet_offset[l + 1] - b;
         if (!n) continue;
         const GridGeom g = T->leaf_geom(int(l), dims, scaling);
-        const int32_t* ids = T->d_pairs.as<int32_t>() + b;
-        double* grid = T->d_grids.as<double>() + l * cells;
-        const hipError_t e = direct_deposit_fits(g, n)
-                                 ? launch_direct_lattice(lv, decomposition, ids, n, g, tet_mass, grid, ctr + l, L->device, ds.stream)
-                                 : launch_deposit_lattice_plain(lv, decomposition, ids, n, g, tet_mass, grid, nullptr, ds.stream);
+        hipError_t e = launch_deposit_lattice_plain(lv, decomposition, T->d_pairs.as<int32_t>() + b, n, g, tet_mass,
+                                                    T->d_grids.as<double>() + l * cells, nullptr, ds.stream);
         if (e != hipSuccess) return hip_fail(e, "leaf deposit launch");
     }
     return ADECO_OK;
@@ -377,14 +372,14 @@ adeco_status adeco_deposit_leaves(adeco_octree T, int dims, int decomposition, d
     g_timings.main_ms = g_last_kernel_ms;
     if (!plain && T->d_fallback) {
         float ms = 0.f;
-        unsigned long long cnt[2] = {0, 0};
+        unsigned long long cnt[3] = {0, 0, 0};  // recomputes, partials, and the direct form's blocks
         e = hipEventElapsedTime(&ms, ds.evk0, ds.evk1);
-        if (e == hipSuccess) e = hipMemcpy(cnt, T->d_fallback, 16, hipMemcpyDeviceToHost);
+        if (e == hipSuccess) e = hipMemcpy(cnt, T->d_fallback, sizeof(cnt), hipMemcpyDeviceToHost);
         if (e != hipSuccess) return hip_fail(e, "batched timings");
         g_timings.main_ms = ms;
         g_timings.fallbacks = double(cnt[0]);
         g_timings.partials = double(cnt[1]);
-        g_timings.candidates = double(T->last_candidates);
+        g_timings.candidates = T->last_candidates < 0 ? double(cnt[2]) : double(T->last_candidates);
     }
     return ADECO_OK;
 }

@@ -11,6 +11,7 @@ import pytest
 import adeco_amd as A
 from tests import _oracle as O
 from tests.test_block_clip import soup_of_extents
+from tests.test_gpu_leaves import make_lattice
 
 pytestmark = pytest.mark.gpu
 BOX = np.array([0, 32, 0, 32, 0, 32], np.float32)
@@ -77,3 +78,22 @@ def test_cells_with_a_sentinel_vertex_deposit_nothing():
     A.DepositWrapper.deposit_tets(True, 0, 0, 3, np.ascontiguousarray(pat).reshape(-1), pat.size, 7, box, 16, data)
     cells = 343 + 3 * 49 + 342
     assert abs(data.astype(np.float64).sum() - 6 * cells) <= 1e-5 * 6 * cells
+
+
+@pytest.mark.parametrize("dims", [2, 5, 10, 24])
+def test_leaves_from_pairs_or_pair_lines(dims):
+    """Batched leaves on either side of 4 pairs per cell, and plain ones, against the captured deposit, which
+    always goes through pair lines."""
+    lat = make_lattice(24, 3.0, seed=9)
+    print(f"[direct] leaves {dims}", flush=True)
+    with A.ResidentLattice.from_lattice(lat) as rl, A.Octree(rl, 1500, 3) as tree:
+        pairs = int(tree.bin(A.DECOMP_KUHN).sum())
+        assert (pairs >= 4 * tree.num_leaves * dims ** 3) == (dims <= 5)
+        with A.DepositGraph(tree, dims, A.DECOMP_KUHN, 0.5, A.PREC_FP64) as g:
+            g.launch()
+            want = g.leaf_grids()
+        for mode in (A.MODE_BATCHED, A.MODE_PLAIN):
+            tree.deposit(dims, A.DECOMP_KUHN, 0.5, mode)
+            got = tree.leaf_grids()
+            assert got.shape == want.shape
+            assert np.abs(got - want).max() <= 1e-12 * want.max()
