@@ -265,9 +265,7 @@ adeco_status adeco_deposit_graph_grids(adeco_deposit_graph G, int64_t first_leaf
     const int64_t cells = int64_t(G->dims) * G->dims * G->dims;
     hipError_t e = hipSetDevice(G->device);
     if (e == hipSuccess)
-        e = hipMemcpyAsync(out, G->grids.as<double>() + first_leaf * cells, size_t(n_leaves * cells) * 8,
-                           hipMemcpyDeviceToHost, G->stream);
-    if (e == hipSuccess) e = hipStreamSynchronize(G->stream);
+        e = download(*G->T->L->ds, G->stream, out, G->grids.as<double>() + first_leaf * cells, size_t(n_leaves * cells) * 8);
     return e == hipSuccess ? ADECO_OK : hip_fail(e, "deposit graph grids");
 }
 

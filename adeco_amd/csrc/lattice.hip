@@ -349,10 +349,8 @@ adeco_status adeco_lattice_deposit_grid(adeco_lattice L, int decomposition, doub
                                          stats ? ds.stats.as<unsigned long long>() : nullptr, ds.stream);
     if (e != hipSuccess) return hip_fail(e, "deposit launch");
     if ((st = timed_end(ds))) return st;
-    e = hipMemcpyAsync(grid_out, ds.grid.ptr, ncell * sizeof(double), hipMemcpyDeviceToHost, ds.stream);
-    if (e == hipSuccess && stats)
-        e = hipMemcpyAsync(stats, ds.stats.ptr, kNumStats * sizeof(unsigned long long), hipMemcpyDeviceToHost, ds.stream);
-    if (e == hipSuccess) e = hipStreamSynchronize(ds.stream);
+    if (stats) e = hipMemcpyAsync(stats, ds.stats.ptr, kNumStats * sizeof(unsigned long long), hipMemcpyDeviceToHost, ds.stream);
+    if (e == hipSuccess) e = download(ds, ds.stream, grid_out, ds.grid.ptr, ncell * sizeof(double));
     if (e != hipSuccess) return hip_fail(e, "deposit download");
     (void)mode;
     (void)precision;
@@ -396,10 +394,8 @@ adeco_status adeco_deposit_soup(int device_id, const float* tets, int64_t n_tets
         if (e != hipSuccess) return hip_fail(e, "soup launch");
     }
     if ((st = timed_end(ds))) return st;
-    e = hipMemcpyAsync(grid_out, ds.grid.ptr, ncell * sizeof(double), hipMemcpyDeviceToHost, ds.stream);
-    if (e == hipSuccess && stats)
-        e = hipMemcpyAsync(stats, ds.stats.ptr, kNumStats * sizeof(unsigned long long), hipMemcpyDeviceToHost, ds.stream);
-    if (e == hipSuccess) e = hipStreamSynchronize(ds.stream);
+    if (stats) e = hipMemcpyAsync(stats, ds.stats.ptr, kNumStats * sizeof(unsigned long long), hipMemcpyDeviceToHost, ds.stream);
+    if (e == hipSuccess) e = download(ds, ds.stream, grid_out, ds.grid.ptr, ncell * sizeof(double));
     if (e != hipSuccess) return hip_fail(e, "soup download");
     return ADECO_OK;
 }

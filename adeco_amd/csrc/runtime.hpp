@@ -54,6 +54,10 @@ struct DeviceState {
     // call on this device (calls hold the mutex)
     DevBuf soup, soup_ids, soup_desc, soup_work, soup_tiles, soup_ctr;
     adeco_status ensure(int dev);
+    // streams of download() (created by its first large copy)
+    static constexpr int kDownloads = 4;
+    std::mutex down_mutex;
+    hipStream_t down[kDownloads] = {};
 };
 
 // A named roctx range over a host scope (rocprofv3 --marker-trace shows it); next() ends it and
@@ -72,6 +76,9 @@ struct TraceRange {
 
 DeviceState& device_state(int dev);
 size_t memory_budget(const DeviceState& ds);
+// Copies what `stream` has computed to the caller's memory and waits for it; a large result in kDownloads
+// parts side by side.
+hipError_t download(DeviceState& ds, hipStream_t stream, void* dst, const void* src, size_t bytes);
 adeco_status timed_begin(DeviceState& ds);
 adeco_status timed_end(DeviceState& ds);
 

@@ -655,8 +655,7 @@ void adeco_server_s::run_copier() {
         lk.unlock();
         // the request's last step and density kernel, then the download
         hipError_t e = hipEventSynchronize(slot_done[r->slot]);
-        if (e == hipSuccess) e = hipMemcpyAsync(r->host_out, s.out32.ptr, bytes, hipMemcpyDeviceToHost, copy_stream);
-        if (e == hipSuccess) e = hipStreamSynchronize(copy_stream);
+        if (e == hipSuccess) e = download(*L->ds, copy_stream, r->host_out, s.out32.ptr, bytes);
         lk.lock();
         if (e != hipSuccess) r->status = hip_fail(e, "request download");
         r->t_done = now_s();
@@ -846,8 +845,7 @@ adeco_status adeco_roi_deposit_plain(adeco_lattice L, int decomposition, double 
     hipLaunchKernelGGL(k_density_f32, dim3(unsigned(std::min<int64_t>((cells + 255) / 256, 4096))), dim3(256), 0, ds.stream,
                        ds.grid.as<double>(), cells, 1.0 / g.cell_vol, ds.scratch.as<float>());
     e = hipGetLastError();
-    if (e == hipSuccess) e = hipMemcpyAsync(density_out, ds.scratch.ptr, size_t(cells) * 4, hipMemcpyDeviceToHost, ds.stream);
-    if (e == hipSuccess) e = hipStreamSynchronize(ds.stream);
+    if (e == hipSuccess) e = download(ds, ds.stream, density_out, ds.scratch.ptr, size_t(cells) * 4);
     if (e != hipSuccess) return hip_fail(e, "roi_deposit_plain() download");
     if (n_tets_out) *n_tets_out = n;
     return ADECO_OK;

@@ -482,7 +482,7 @@ adeco_status adeco_leaf_grids(adeco_octree T, int64_t first_leaf, int64_t n_leav
     std::lock_guard<std::mutex> lk(T->L->ds->mutex);
     hipError_t e = hipSetDevice(T->L->device);
     if (e == hipSuccess)
-        e = hipMemcpy(out, T->d_grids.as<double>() + first_leaf * cells, size_t(n_leaves * cells) * 8, hipMemcpyDeviceToHost);
+        e = download(*T->L->ds, T->L->ds->stream, out, T->d_grids.as<double>() + first_leaf * cells, size_t(n_leaves * cells) * 8);
     return e == hipSuccess ? ADECO_OK : hip_fail(e, "leaf grid download");
 }
 

@@ -97,3 +97,17 @@ def test_leaves_from_pairs_or_pair_lines(dims):
             got = tree.leaf_grids()
             assert got.shape == want.shape
             assert np.abs(got - want).max() <= 1e-12 * want.max()
+
+
+@pytest.mark.parametrize("dims", [101, 102, 131])
+def test_results_around_the_split_download(dims):
+    """Grids just below and above 8 MiB (one copy, four side by side, no whole number of pages each)."""
+    rng = np.random.default_rng(dims)
+    tets = (soup_of_extents(rng, [(1, 2, 2), (3, 3, 2)], 60).astype(np.float64) * (dims / 32.0)).astype(np.float32)
+    box = np.array([0, dims] * 3, np.float32)
+    print(f"[direct] download {dims}", flush=True)
+    got = A.deposit_soup(tets, box, dims, 1.0)
+    with O.cell_scaling(O.EXACT):
+        want = O.deposit_soup_ld(tets, box, dims, 1.0)
+    assert all(part.sum() > 0 for part in np.array_split(want, 4))
+    assert O.max_rel_err(got, want, tet_mass=1.0) <= 1e-6
