@@ -133,11 +133,21 @@ struct Rows {
     bool both;
 };
 
+// The same for a row and a column of cells: the index of the first cell of column yr in row xr, and the steps
+// to the next column and row (0: not counted there), in a block of cy columns of cz cells.
+struct Target {
+    int base, dy, dx, cz;
+    ADECO_HD Target() {}
+    ADECO_HD Target(Rows xr, Rows yr, int cy, int cz_)
+        : base((xr.at * cy + yr.at) * cz_), dy(yr.both ? cz_ : 0), dx(xr.both ? cy * cz_ : 0), cz(cz_) {}
+};
+
 // Adds the shares of a piece with heights z0..z3 (any order) and signed share w between the z planes
-// 0..cz, cell by cell, in the rows xr and columns yr (of cy).  Without branches but for the loop over the
-// planes that cut it: an add that does not apply adds 0 to the same cell.
+// 0..cz, cell by cell, where t says.  Without branches but for the loop over the planes that cut it: an add
+// that does not apply adds 0 to the same cell.  Acc: term(share) a value to sum (with its negative), add(cell,
+// value).
 template <class Acc>
-ADECO_HD void block_leaf(double z0, double z1, double z2, double z3, double w, Rows xr, Rows yr, int cy, int cz, Acc& acc) {
+ADECO_HD void block_leaf(double z0, double z1, double z2, double z3, double w, Target t, Acc& acc) {
 #define ADECO_MINMAX(u, v)        \
     {                             \
         const double lo_ = fmin(u, v); \
@@ -147,19 +157,18 @@ ADECO_HD void block_leaf(double z0, double z1, double z2, double z3, double w, R
     ADECO_MINMAX(z0, z1) ADECO_MINMAX(z2, z3) ADECO_MINMAX(z0, z2) ADECO_MINMAX(z1, z3) ADECO_MINMAX(z1, z2)
 #undef ADECO_MINMAX
     // planes first..last cut the piece
-    const int first = floor_clamped(z0, cz) + 1, last = ceil_clamped(z3, cz) - 1;
-    const int base = (xr.at * cy + yr.at) * cz;
-    const int by = base + (yr.both ? cz : 0), bx = base + (xr.both ? cy * cz : 0), bxy = bx + (yr.both ? cz : 0);
+    const int first = floor_clamped(z0, t.cz) + 1, last = ceil_clamped(z3, t.cz) - 1;
+    const int base = t.base, by = base + t.dy, bx = base + t.dx, bxy = bx + t.dy;
     const double d20 = z2 - z0, d30 = z3 - z0, d31 = z3 - z1;
     const double D1 = (z1 - z0) * d20 * d30, D2 = d20 * d30 * (z2 - z1) * d31, D3 = d30 * d31 * (z3 - z2);
     double prev = 0.0;
     int h = first;
     const auto emit = [&](int k, double v) {
-        const double vy = yr.both ? -v : 0.0, vx = xr.both ? -v : 0.0, vxy = yr.both ? -vx : 0.0;
-        acc.add(base + k, v);
-        acc.add(by + k, vy);
+        const auto u = acc.term(v), zero = u - u, vx = t.dx ? -u : zero;
+        acc.add(base + k, u);
+        acc.add(by + k, t.dy ? -u : zero);
         acc.add(bx + k, vx);
-        acc.add(bxy + k, vxy);
+        acc.add(bxy + k, t.dy ? -vx : zero);
     };
     for (; h <= last; ++h) {
         const double zh = double(h);
@@ -176,14 +185,26 @@ ADECO_HD void block_leaf(double z0, double z1, double z2, double z3, double w, R
         prev = below;
     }
     // the cell above the last plane, or the piece's only cell
-    const bool top = last < cz && z3 > 0.0 && z0 < double(cz);
+    const bool top = last < t.cz && z3 > 0.0 && z0 < double(t.cz);
     emit(top ? h - 1 : 0, top ? w * (1.0 - prev) : 0.0);
 }
 
-// One piece (y, z at its vertices, any order; signed share w) against the y planes 0..cy.
+// Takes the leaves (pieces of both cuts) of block_shares as they come.  On the device one that gathers them over
+// the lanes of a wave takes its place, whose loops therefore go on while any lane has work: any(b) is true if b
+// is for any of them.
 template <class Acc>
-ADECO_HD void block_piece(double y0, double y1, double y2, double y3, double z0, double z1, double z2, double z3, double w,
-                          Rows xr, int cy, int cz, Acc& acc) {
+struct LeafSums {
+    Acc& acc;
+    ADECO_HD bool any(bool b) const { return b; }
+    ADECO_HD void leaf(bool on, double z0, double z1, double z2, double z3, double w, Target t) {
+        if (on) block_leaf(z0, z1, z2, z3, w, t, acc);
+    }
+};
+
+// One piece (y, z at its vertices, any order; signed share w) against the y planes 0..cy.
+template <class Leaves>
+ADECO_HD void block_piece(bool on, double y0, double y1, double y2, double y3, double z0, double z1, double z2, double z3, double w,
+                          Rows xr, int cy, int cz, Leaves& leaves) {
     order2(y0, y1, z0, z1);
     order2(y2, y3, z2, z3);
     order2(y0, y2, z0, z2);
@@ -191,7 +212,7 @@ ADECO_HD void block_piece(double y0, double y1, double y2, double y3, double z0,
     order2(y1, y2, z1, z2);
     PlaneRange r;
     r.set(y0, y2, y3, cy);
-    for (int q = r.whole < cy ? r.first - 1 : r.first; q <= r.last; ++q) {
+    for (int q = r.whole < cy ? r.first - 1 : r.first; leaves.any(on && q <= r.last); ++q) {
         // the piece itself, or what the cut by plane q leaves below it
         const bool t = q < r.first;
         ADECO_KEEP_IN_LOOP(y0);
@@ -207,11 +228,12 @@ ADECO_HD void block_piece(double y0, double y1, double y2, double y3, double z0,
         double g0 = !t && e.three ? z3 : z0;
         const double g3 = t || (!e.one && !e.three) ? z1 : hC;
         double s = t ? w : (q > 0 ? w : -w) * e.w0;
-        const int np = t ? 1 : e.pieces();
+        const int np = on && q <= r.last ? (t ? 1 : e.pieces()) : 0;
         const Rows yr{t ? r.whole : (q > 0 ? q - 1 : 0), !t && q > 0 && q < cy};
+        const Target at(xr, yr, cy, cz);
         for (int k = 0;;) {
-            block_leaf(g0, hA, hB, g3, s, xr, yr, cy, cz, acc);
-            if (++k >= np) break;
+            leaves.leaf(k < np, g0, hA, hB, g3, s, at);
+            if (!leaves.any(++k < np)) break;
             hB = k == 2 ? hC : hB;
             g0 = hD;
             s = (q > 0 ? w : -w) * (k == 1 ? e.w1 : e.w2);
@@ -219,10 +241,11 @@ ADECO_HD void block_piece(double y0, double y1, double y2, double y3, double z0,
     }
 }
 
-// Adds to acc (index (a * cy + b) * cz + k) the share of the tet (vertices x, y, z in cells from the
-// block's corner) in every cell of the block.  cx * cy * cz <= kBlockCells.
-template <class Acc>
-ADECO_HD void block_shares(const double x[4], const double y[4], const double z[4], int cx, int cy, int cz, Acc& acc) {
+// Gives `leaves` the pieces of the tet (vertices x, y, z in cells from the block's corner) that sum to its share
+// in every cell of the block (index (a * cy + b) * cz + k).  cx * cy * cz <= kBlockCells.  on: there is a tet.
+template <class Leaves>
+ADECO_HD void block_shares(bool on, const double x[4], const double y[4], const double z[4], int cx, int cy, int cz,
+                           Leaves& leaves) {
     double x0 = x[0], x1 = x[1], x2 = x[2], x3 = x[3];
     double y0 = y[0], y1 = y[1], y2 = y[2], y3 = y[3];
     double z0 = z[0], z1 = z[1], z2 = z[2], z3 = z[3];
@@ -233,7 +256,7 @@ ADECO_HD void block_shares(const double x[4], const double y[4], const double z[
     order3(x1, x2, y1, y2, z1, z2);
     PlaneRange r;
     r.set(x0, x2, x3, cx);
-    for (int p = r.whole < cx ? r.first - 1 : r.first; p <= r.last; ++p) {
+    for (int p = r.whole < cx ? r.first - 1 : r.first; leaves.any(on && p <= r.last); ++p) {
         // the tet itself, or the pieces of the part below plane p
         const bool t = p < r.first;
         ADECO_KEEP_IN_LOOP(x0);
@@ -253,11 +276,11 @@ ADECO_HD void block_shares(const double x[4], const double y[4], const double z[
         double py2 = t ? y2 : e.atB(y0, y1, y2, y3), pz2 = t ? z2 : e.atB(z0, z1, z2, z3);
         const double py3 = t || two ? y1 : cy_, pz3 = t || two ? z1 : cz_;
         double w = t ? 1.0 : (p > 0 ? e.w0 : -e.w0);
-        const int np = t ? 1 : e.pieces();
+        const int np = on && p <= r.last ? (t ? 1 : e.pieces()) : 0;
         const Rows xr{t ? r.whole : (p > 0 ? p - 1 : 0), !t && p > 0 && p < cx};
         for (int k = 0;;) {
-            block_piece(py0, py1, py2, py3, pz0, pz1, pz2, pz3, w, xr, cy, cz, acc);
-            if (++k >= np) break;
+            block_piece(k < np, py0, py1, py2, py3, pz0, pz1, pz2, pz3, w, xr, cy, cz, leaves);
+            if (!leaves.any(++k < np)) break;
             py2 = k == 2 ? cy_ : py2;
             pz2 = k == 2 ? cz_ : pz2;
             py0 = dy_;

@@ -10,19 +10,21 @@
 //                       plane of the tet separates from it are dropped, blocks inside it are filled, and
 //                       the others go to one of 6 per-wave LDS queues by the number of x and y planes
 //                       that cut the tet, so that the 64 lanes of a pass run through similar loops.  A
-//                       full queue is clipped by the whole wave: each lane sums its block's shares in
-//                       LDS (one column of kBlockCells doubles per lane) and adds tet_mass * share to
-//                       the grid.  A share too small against the differences' rounding goes to one more
-//                       queue whose passes recompute that cell alone from positive terms.
+//                       full queue is clipped by the whole wave: each lane cuts its block's tet, the
+//                       pieces are summed one per lane into their blocks' LDS columns, and each lane adds
+//                       tet_mass * share to the grid.  A share too small against the differences'
+//                       rounding goes to one more queue whose passes recompute that cell alone from
+//                       positive terms.
 // Why blocks: the column form clips every column of a tet on its own, so a tet of 2 x 2 columns is cut by
 // each inner plane twice over and through up to four nested stages of full 3-D pieces.  Here a plane is
 // cut once for the cells on both its sides, a cut carries only the coordinates still needed and a
-// piece's volume comes from edge ratios (4-5x fewer instructions per tet, 168 VGPRs: 3 waves per SIMD
-// instead of 2).  256^3 clustered lattice, 16^3-cell leaves, 126 M pairs: 31.4 ms against 65.6 for the
-// column form; 128^3: 3.8 against 7.1; 32^3-cell leaves on 97^3: 15.3 against 27.5.  It is also more
-// accurate (128^3 leaf grids against 64-bit exact clipping: 9e-15 against 3e-13).  What bounds it:
-// instruction issue at 40-50 % lane use, then FP64 atomics (one per cell a tet meets; the card takes
-// 25-31 G/s of them scattered).
+// piece's volume comes from edge ratios (4-5x fewer instructions per tet).  256^3 clustered lattice,
+// 16^3-cell leaves, 126 M pairs: 31.4 ms against 65.6 for the column form; 128^3: 3.8 against 7.1;
+// 32^3-cell leaves on 97^3: 15.3 against 27.5, and 10.8 with the pieces gathered over the lanes
+// (block_wave.hpp).  It is also more accurate (128^3 leaf grids against 64-bit exact clipping: 4e-15
+// against 2e-13).  What bounds it: instruction issue at 40-60 % lane use, then FP64 atomics (one per cell a
+// tet meets; the card takes 25-31 G/s of them scattered).  Two workgroups of 4 waves per CU: 20 KB of LDS a
+// wave, and no spills (205 VGPRs; at 168 and 3 workgroups about 45 are spilled around each pass).
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -45,7 +47,7 @@ constexpr int kCells = 16;
 using Lds = BlockLds<kCells>;
 
 // 3 workgroups of 4 waves share the 160 KB of a CU, which are handed out in pieces of 1280 bytes
-static_assert((sizeof(Lds) * kWaves + 1279) / 1280 * 1280 * 3 <= 160 * 1024, "3 workgroups per CU");
+static_assert((sizeof(Lds) * kWaves + 1279) / 1280 * 1280 * 2 <= 160 * 1024, "2 workgroups per CU");
 
 // A queue entry: the pair, and the block's index in it with the source slot in the upper 6 bits (a
 // pair has at most 512 * 512 * 256 = 2^26 blocks).
@@ -226,7 +228,7 @@ __device__ __forceinline__ void deposit_tiles(const Sources& srcs, const int2* _
     if (w.n_exact) atomicAdd(counters, (unsigned long long)w.n_exact);
 }
 
-__global__ void __launch_bounds__(kThreads, 3) k_deposit_blocks(TileSource src, int chunk, unsigned* __restrict__ queue_counter,
+__global__ void __launch_bounds__(kThreads, 2) k_deposit_blocks(TileSource src, int chunk, unsigned* __restrict__ queue_counter,
                                                                 unsigned long long* __restrict__ counters) {
     if (src.dev_sizes) {
         src.n_cand = src.dev_sizes[0];
@@ -235,7 +237,7 @@ __global__ void __launch_bounds__(kThreads, 3) k_deposit_blocks(TileSource src, 
     deposit_tiles(OneSource{src}, nullptr, src.n_tiles, chunk, queue_counter, counters);
 }
 
-__global__ void __launch_bounds__(kThreads, 3) k_step_blocks(const TileSource* __restrict__ sources,
+__global__ void __launch_bounds__(kThreads, 2) k_step_blocks(const TileSource* __restrict__ sources,
                                                              const int2* __restrict__ entries, int n_entries, int chunk,
                                                              unsigned* __restrict__ queue_counter,
                                                              unsigned long long* __restrict__ counters) {
@@ -245,6 +247,7 @@ __global__ void __launch_bounds__(kThreads, 3) k_step_blocks(const TileSource* _
 // This tet's shares on the host (the same code; tests only).
 struct HostShares {
     double* a;
+    static double term(double share) { return share; }
     void add(int i, double v) { a[i] += v; }
 };
 
@@ -300,7 +303,8 @@ extern "C" int adeco_selftest_block_f64(const double* t, const int* cells3, doub
     }
     for (int i = 0; i < n; ++i) shares[i] = 0.0;
     HostShares sum{shares};
-    block_shares(x, y, z, cx, cy, cz, sum);
+    LeafSums<HostShares> leaves{sum};
+    block_shares(true, x, y, z, cx, cy, cz, leaves);
     for (int i = 0; i < n; ++i) {
         const int k = i % cz, b = (i / cz) % cy, a = i / (cz * cy);
         double lx[4], ly[4], lz[4], keep[15];

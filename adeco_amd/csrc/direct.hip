@@ -8,9 +8,9 @@
 // and full queues are clipped by the whole wave.  So a wave's lanes share the cells of a large tet, and
 // nothing but the tets is read from memory.
 // Against the one-tet-per-thread kernel (deposit.hip), whose waves run as long as their largest tet
-// walks its cells: one meta-patch of 2 058 tets on 16^3 cells 120 us against 900-1130, a leaf's 98 784 tets
-// on 16^3 cells 215 against 1420-1530, 196 608 tets on 64^3 cells 0.43 ms against 3.8.  All leaves of an
-// octree in one launch instead of one each: 64 leaves, 1.86 M pairs, 16^3 cells 0.77 ms against 15.2.
+// walks its cells: one meta-patch of 2 058 tets on 16^3 cells 104 us against 900-1130, a leaf's 98 784 tets
+// on 16^3 cells 172 against 1420-1530, 196 608 tets on 64^3 cells 0.31 ms against 3.8.  All leaves of an
+// octree in one launch instead of one each: 64 leaves, 1.86 M pairs, 16^3 cells 0.66 ms against 15.2.
 // What bounds it: a small launch lasts as long as one wave's chain of passes (classify, clip, recompute:
 // 20-30 us each, at mostly one wave per SIMD); a large one is bound as the batched form is (blocks.hip).
 #include <hip/hip_runtime.h>
@@ -33,7 +33,7 @@ constexpr int kWaves = 4;
 constexpr int kThreads = 64 * kWaves;
 constexpr int kCells = 16;
 using Lds = BlockLds<kCells>;
-static_assert((sizeof(Lds) * kWaves + 1279) / 1280 * 1280 * 3 <= 160 * 1024, "3 workgroups per CU");
+static_assert((sizeof(Lds) * kWaves + 1279) / 1280 * 1280 * 2 <= 160 * 1024, "2 workgroups per CU");
 
 // Tets of one grid.
 struct OneGrid {
@@ -249,7 +249,7 @@ struct DirectFeed {
 };
 
 template <class Tets>
-__global__ void __launch_bounds__(kThreads, 3) k_deposit_direct(Tets tets, unsigned n_tets, unsigned per_item, unsigned per_pop,
+__global__ void __launch_bounds__(kThreads, 2) k_deposit_direct(Tets tets, unsigned n_tets, unsigned per_item, unsigned per_pop,
                                                                 double tet_mass, double* __restrict__ grid,
                                                                 DirectCounters* __restrict__ ctr) {
     __shared__ Lds lds[kWaves];
@@ -273,7 +273,7 @@ hipError_t launch(const Tets& tets, int64_t n_tets, int dims, bool small_tets, d
     // tets per item: 64 fill a wave's lanes; fewer where that leaves resident waves without work (a small
     // launch is over when its slowest wave is, and large tets bring many blocks each): about two items
     // per resident wave
-    const int64_t waves = int64_t(cus) * 3 * kWaves;
+    const int64_t waves = int64_t(cus) * 2 * kWaves;
     // (64 tets of up to 2^26 blocks each would overflow their 32-bit sum on grids beyond 512^3)
     int per_item = dims <= 512 ? 64 : 32;
     while (per_item > 1 && n_tets < 2 * waves * per_item) per_item >>= 1;
