@@ -22,8 +22,8 @@
 
 namespace adeco {
 
-// Largest number of cells in a block (a kernel may take smaller ones).
-constexpr int kBlockCells = 16;
+// Largest number of cells in a block.
+constexpr int kBlockCells = 24;
 // Shares of a cell below kNoShare (18 ulps of the tet: the differences' rounding) are empty; between
 // that and kSmallShare they are recomputed by exact_cell_share.
 constexpr double kNoShare = 4e-15;

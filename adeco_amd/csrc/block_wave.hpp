@@ -15,16 +15,15 @@
 
 namespace adeco {
 
-constexpr int kClasses = 6;            // queues of blocks to clip
+constexpr int kClasses = 8;            // queues of blocks to clip
 constexpr int kExact = kClasses;       // the queue of single cells to recompute
 constexpr int kQueues = kClasses + 1;
+static_assert(kClasses <= 8 && kQueues <= 16, "the drain's prefix sum and the counts");
 
-// Per-wavefront LDS for blocks of up to E cells.  A queue entry is an int2 that the kernel's loader
+// Per-wavefront LDS.  A queue entry is an int2 that the kernel's loader
 // understands.  An entry that finds its queue full is carried per lane and takes its place once that
 // queue has been clipped; qn[b] counts queue b's entries and its carried ones.
-template <int E>
 struct BlockLds {
-    static_assert(E >= 15, "exact_cell_share keeps 15 values in a lane's column");
     int qn[16];
     int2 q[kQueues][kWaveTile];
     int2 carry[kWaveTile];
@@ -33,39 +32,42 @@ struct BlockLds {
     double leaf[5][kWaveTile];      // leaves of the pass: 4 heights and the share,
     unsigned leaf_to[kWaveTile];    // and where they count
     union {
-        unsigned long long sum[E][kWaveTile];  // each lane's shares, in units of 2^-62
-        double keep[E][kWaveTile];             // each lane's storage of a recompute
+        unsigned long long sum[kBlockCells][kWaveTile];  // each lane's shares, in units of 2^-62
+        double keep[15][kWaveTile];             // each lane's storage of a recompute
         int mark[kWaveTile];       // starts of the tile being classified
     };
 };
 
 // How covered cells are cut into blocks: blocks of b cells, n of them, per axis (x, y, z in the pair's
-// order, extents ex <= ey <= ez).  A cover of at most E cells is one block; else x keeps up to 2 cells, z
-// up to 4 (3 of E = 12) and y what is left, the cells spread evenly over an axis' blocks.
+// order, extents ex <= ey <= ez).  A cover of at most kBlockCells cells is one block; else x keeps up to 2 cells,
+// z up to 6 (more where x and y have few) and y what is left, the cells spread evenly over an axis' blocks.
+// Large blocks cut fewer faces between blocks, and planes across z cost least.  24 cells are what the LDS of a
+// wave holds; against 16 (2 x 2 x 4): 15.3 M pairs on 16^3-cell leaves 4.02 -> 3.71 ms, 6.7 M pairs on
+// 32^3-cell leaves 10.9 -> 9.75, a request of 200^3 cells 515 -> 409 us.
 struct BlockShape {
     int b[3], n[3];
 };
 
-template <int E>
 __device__ __forceinline__ BlockShape block_shape(int ex, int ey, int ez) {
-    static_assert(E == 12 || E == 16, "block sizes");
+    static_assert(kBlockCells == 24, "block sizes");
+    const int e[3] = {ex, ey, ez};
     BlockShape s;
-    s.b[0] = ex;
-    s.b[1] = ey;
-    s.b[2] = ez;
-    s.n[0] = s.n[1] = s.n[2] = 1;
-    if (ex * ey * ez <= E) return s;
-    const int bz = min(ez, E / 4);
-    const int bx = min(ex, 2), xz = bx * bz;
-    // E / (bx * bz) for the products that occur (1-4, 6, 8)
-    const int room = E == 16 ? (xz <= 2 ? 8 : (xz == 3 ? 5 : (xz == 4 ? 4 : 2))) : (xz <= 2 ? 6 : (xz == 3 ? 4 : (xz == 4 ? 3 : 2)));
-    const int b[3] = {bx, min(ey, room), bz};
-    for (int a = 0; a < 3; ++a)
-        if (b[a] < s.b[a]) {
-            const int e = s.b[a], n = int(udiv_small(unsigned(e + b[a] - 1), unsigned(b[a])));
-            s.b[a] = int(udiv_small(unsigned(e + n - 1), unsigned(n)));
-            s.n[a] = int(udiv_small(unsigned(e + s.b[a] - 1), unsigned(s.b[a])));
-        }
+    for (int a = 0; a < 3; ++a) {
+        s.b[a] = e[a];
+        s.n[a] = 1;
+    }
+    if (ex * ey * ez <= kBlockCells) return s;
+    const auto cut = [&](int a, int most) {
+        if (e[a] <= most) return;
+        const int n = int(udiv_small(unsigned(e[a] + most - 1), unsigned(most)));
+        s.b[a] = int(udiv_small(unsigned(e[a] + n - 1), unsigned(n)));
+        s.n[a] = int(udiv_small(unsigned(e[a] + s.b[a] - 1), unsigned(s.b[a])));
+    };
+    cut(0, 2);
+    const int xy = s.b[0] * min(ey, 4);
+    cut(2, xy == 1 ? 24 : (xy == 2 ? 12 : (xy == 3 ? 8 : 6)));
+    // 24 / (x * z): the quotient is at least 0.02 from the next whole number
+    cut(1, int(24.5f * __builtin_amdgcn_rcpf(float(s.b[0] * s.b[2]))));
     return s;
 }
 
@@ -105,10 +107,9 @@ struct Block {
 };
 
 // lo, e: the cover's first cell and extents in its axis order; s: the vertices in cells, in that order.
-template <int E>
 __device__ __forceinline__ Block make_block(const int lo[3], const int e[3], const double s[4][3], unsigned unit) {
     Block b;
-    const BlockShape sh = block_shape<E>(e[0], e[1], e[2]);
+    const BlockShape sh = block_shape(e[0], e[1], e[2]);
     int i[3] = {0, 0, 0};
     if (unit) {
         const unsigned rest = sh.n[2] == 1 ? unit : udiv_small(unit, unsigned(sh.n[2]));
@@ -164,18 +165,22 @@ __device__ __forceinline__ void for_cells(const int c[3], const Place& p, F f) {
     }
 }
 
-// Work class of a block to clip: by the planes that cut the tet across x and y, and for a single x plane
-// by whether it leaves one piece (1 or 3 vertices below) or three.  The class only groups blocks of
-// similar loops.  mn, mx: the tet's extents from the block's corner.
+// Work class of a block to clip: by the pieces that the x planes leave of the tet (1 for each plane with 1 or 3
+// vertices below, else 3), and where they are few by the planes that cut it across y.  The class only groups
+// blocks of similar loops (8 classes against 6 by the planes alone: 9.75 -> 9.2 ms for the large tets above,
+// 3.71 -> 3.68 for the small ones).  mn, mx: the tet's extents from the block's corner.
 __device__ __forceinline__ int work_class(const Block& b, const double mn[3], const double mx[3]) {
     const int fx = floor_clamped(mn[0], b.c[0]) + 1, lx = min(ceil_clamped(mx[0], b.c[0]) - 1, b.c[0]);
     const int fy = floor_clamped(mn[1], b.c[1]) + 1, ly = min(ceil_clamped(mx[1], b.c[1]) - 1, b.c[1]);
-    const int px = lx - fx + 1, py = ly - fy + 1;
-    if (px <= 0) return 0;
-    if (px >= 2) return 5;
-    int n = 0;
-    for (int q = 0; q < 4; ++q) n += int(b.x[q] < double(fx));
-    return (py <= 1 ? 1 : 3) + int(n == 2);
+    const int py = ly - fy + 1;
+    int pieces = 0;
+    for (int p = 0; p <= 2; ++p) {  // (a block has at most 2 cells across x)
+        const int n = int(b.x[0] < double(p)) + int(b.x[1] < double(p)) + int(b.x[2] < double(p)) + int(b.x[3] < double(p));
+        pieces += p >= fx && p <= lx ? (n == 2 ? 3 : 1) : 0;
+    }
+    if (pieces <= 1) return 2 * pieces + int(py > pieces);
+    if (pieces == 3) return 5 + int(py > 1);
+    return pieces == 2 ? 4 : 7;
 }
 
 enum BlockClass : int { kBlockEmpty = -1, kBlockTet = -2, kBlockFull = -3 };
@@ -213,8 +218,7 @@ __device__ __forceinline__ int mbcnt64(unsigned long long m) {
 
 // Appends each lane's entry to queue `key` (none when key < 0).  Every queue holds < 64 entries before,
 // so a count reaches at most 127; an entry beyond 64 is carried.
-template <int E>
-__device__ __forceinline__ void push_blocks(BlockLds<E>& L, int lane, int key, int2 entry) {
+__device__ __forceinline__ void push_blocks(BlockLds& L, int lane, int key, int2 entry) {
     int ckey = -1;
     if (key >= 0) {
         const int pos = atomicAdd(&L.qn[key], 1);
@@ -249,9 +253,8 @@ struct LaneShares {
 // them, on average a quarter of the lanes had one (large tets; 45 M blocks on 32^3-cell leaves 15.3 ms against
 // 10.8, 196 608 tets on 64^3 cells 430 us against 314; one-block tets, of 3 leaves each, 4.26 ms against 4.02
 // for 15.3 M pairs).
-template <int E>
 struct LeafQueue {
-    BlockLds<E>& L;
+    BlockLds& L;
     int lane;
     int n = 0;  // leaves waiting, < 64
     __device__ __forceinline__ bool any(bool b) const { return __ballot(b) != 0ull; }
@@ -261,17 +264,17 @@ struct LeafQueue {
         L.leaf[2][at] = z2;
         L.leaf[3][at] = z3;
         L.leaf[4][at] = w;
-        L.leaf_to[at] = unsigned(lane) | unsigned(t.base) << 6 | unsigned(t.dy) << 10 | unsigned(t.dx) << 15 | unsigned(t.cz) << 20;
+        L.leaf_to[at] = unsigned(lane) | unsigned(t.base) << 6 | unsigned(t.dy) << 11 | unsigned(t.dx) << 16 | unsigned(t.cz) << 21;
     }
     __device__ __forceinline__ void sum(int count) {
         wave_sync();
         if (lane < count) {
             const unsigned to = L.leaf_to[lane];
             Target t;
-            t.base = int(to >> 6) & 15;
-            t.dy = int(to >> 10) & 31;
-            t.dx = int(to >> 15) & 31;
-            t.cz = int(to >> 20);
+            t.base = int(to >> 6) & 31;
+            t.dy = int(to >> 11) & 31;
+            t.dx = int(to >> 16) & 31;
+            t.cz = int(to >> 21);
             LaneShares acc{&L.sum[0][to & 63u]};
             block_leaf(L.leaf[0][lane], L.leaf[1][lane], L.leaf[2][lane], L.leaf[3][lane], L.leaf[4][lane], t, acc);
         }
@@ -294,11 +297,11 @@ struct LeafQueue {
 // the rounding of the differences: returns their mask (bit = index of the cell in the block).
 // Loader: block(entry) the block, place(entry, lo) the place of a cell of it in its grid (looked up again
 // after the clip, which needs the registers), add(entry, offset, share) the deposit.
-template <int E, class Loader>
-__device__ __forceinline__ unsigned clip_blocks(const Loader& ld, bool on, int2 e, const Block& b, BlockLds<E>& L, int lane) {
+template <class Loader>
+__device__ __forceinline__ unsigned clip_blocks(const Loader& ld, bool on, int2 e, const Block& b, BlockLds& L, int lane) {
     unsigned long long* sum = &L.sum[0][lane];
-    for (int i = 0; i < E; ++i) sum[i * kWaveTile] = 0ull;
-    LeafQueue<E> leaves{L, lane};
+    for (int i = 0; i < kBlockCells; ++i) sum[i * kWaveTile] = 0ull;
+    LeafQueue leaves{L, lane};
     block_shares(on, b.x, b.y, b.z, b.c[0], b.c[1], b.c[2], leaves);
     leaves.sum(leaves.n);
     unsigned redo = 0u;
@@ -336,8 +339,7 @@ struct WaveState {
     unsigned n_exact = 0, n_partial = 0;  // this lane's recomputes, the wave's clipped blocks
 };
 
-template <int E>
-__device__ __forceinline__ void init_wave(BlockLds<E>& L, int lane) {
+__device__ __forceinline__ void init_wave(BlockLds& L, int lane) {
     if (lane < 16) L.qn[lane] = 0;
     L.carry_key[lane] = -1;
     wave_sync();
@@ -347,8 +349,8 @@ __device__ __forceinline__ void init_wave(BlockLds<E>& L, int lane) {
 // `drain`, until the queues are empty: passes filled across the classes, a full queue or the exact one
 // first.  Without `drain` every queue is left below 64 entries and nothing is carried.  A pass takes at
 // least one entry and exact passes add none, so the loop ends.
-template <int E, class Feed, class Loader>
-__device__ __forceinline__ void run_wave(BlockLds<E>& L, int lane, WaveState& w, Feed& feed, const Loader& ld, bool drain) {
+template <class Feed, class Loader>
+__device__ __forceinline__ void run_wave(BlockLds& L, int lane, WaveState& w, Feed& feed, const Loader& ld, bool drain) {
     bool draining = false;
     for (;;) {
         // pending cells go to the exact queue, one per lane and round, up to its 64 entries; a full exact
@@ -448,8 +450,7 @@ __device__ __forceinline__ void run_wave(BlockLds<E>& L, int lane, WaveState& w,
 
 // Tile of 64 consecutive units over items of `cnt` units each (this lane's item: [start, start + cnt)):
 // the item of unit `cursor + lane`, or -1 beyond the last.
-template <int E>
-__device__ __forceinline__ int item_of_unit(BlockLds<E>& L, int lane, unsigned start, unsigned cnt, unsigned cursor) {
+__device__ __forceinline__ int item_of_unit(BlockLds& L, int lane, unsigned start, unsigned cnt, unsigned cursor) {
     L.mark[lane] = -1;
     wave_sync();
     if (cnt > 0 && start < cursor + kWaveTile && start + cnt > cursor) L.mark[int(max(start, cursor) - cursor)] = lane;

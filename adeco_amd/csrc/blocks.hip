@@ -8,8 +8,8 @@
 //   2. scan, tile map   as for the column form (batched.hip);
 //   3. k_deposit_blocks persistent wavefronts pop chunks of tiles of 64 blocks.  Blocks that a face
 //                       plane of the tet separates from it are dropped, blocks inside it are filled, and
-//                       the others go to one of 6 per-wave LDS queues by the number of x and y planes
-//                       that cut the tet, so that the 64 lanes of a pass run through similar loops.  A
+//                       the others go to one of 8 per-wave LDS queues by the pieces that the x and y
+//                       planes make, so that the 64 lanes of a pass run through similar loops.  A
 //                       full queue is clipped by the whole wave: each lane cuts its block's tet, the
 //                       pieces are summed one per lane into their blocks' LDS columns, and each lane adds
 //                       tet_mass * share to the grid.  A share too small against the differences'
@@ -20,10 +20,11 @@
 // cut once for the cells on both its sides, a cut carries only the coordinates still needed and a
 // piece's volume comes from edge ratios (4-5x fewer instructions per tet).  256^3 clustered lattice,
 // 16^3-cell leaves, 126 M pairs: 31.4 ms against 65.6 for the column form; 128^3: 3.8 against 7.1;
-// 32^3-cell leaves on 97^3: 15.3 against 27.5, and 10.8 with the pieces gathered over the lanes
-// (block_wave.hpp).  It is also more accurate (128^3 leaf grids against 64-bit exact clipping: 4e-15
-// against 2e-13).  What bounds it: instruction issue at 40-60 % lane use, then FP64 atomics (one per cell a
-// tet meets; the card takes 25-31 G/s of them scattered).  Two workgroups of 4 waves per CU: 20 KB of LDS a
+// 32^3-cell leaves on 97^3: 15.3 against 27.5, and 9.2 with the pieces gathered over the lanes and blocks of
+// 24 cells (block_wave.hpp).  It is also more accurate (128^3 leaf grids against 64-bit exact clipping:
+// 5e-15 against 2e-13).  What bounds it: vector instructions (issued 80 % of the time with large tets, 55 %
+// with small ones) at 65-75 % lane use, and FP64 atomics (one per cell a tet meets; the card takes 25-31 G/s
+// of them scattered).  Two workgroups of 4 waves per CU: 20 KB of LDS a
 // wave, and no spills (205 VGPRs; at 168 and 3 workgroups about 45 are spilled around each pass).
 #include <hip/hip_runtime.h>
 
@@ -43,11 +44,9 @@ namespace {
 
 constexpr int kWaves = 4;  // wavefronts of a workgroup
 constexpr int kThreads = 64 * kWaves;
-constexpr int kCells = 16;
-using Lds = BlockLds<kCells>;
 
 // 3 workgroups of 4 waves share the 160 KB of a CU, which are handed out in pieces of 1280 bytes
-static_assert((sizeof(Lds) * kWaves + 1279) / 1280 * 1280 * 2 <= 160 * 1024, "2 workgroups per CU");
+static_assert((sizeof(BlockLds) * kWaves + 1279) / 1280 * 1280 * 2 <= 160 * 1024, "2 workgroups per CU");
 
 // A queue entry: the pair, and the block's index in it with the source slot in the upper 6 bits (a
 // pair has at most 512 * 512 * 256 = 2^26 blocks).
@@ -88,7 +87,7 @@ __global__ void __launch_bounds__(256) k_block_setup(LatticeView lat, PackedCorn
         const bool swap = code & 4;
         const int ax = role_axis(code, 0), ay = role_axis(code, 1), za = code & 3;
         const int ex = pick(ax, ext[0], ext[1], ext[2]), ey = pick(ay, ext[0], ext[1], ext[2]), ez = pick(za, ext[0], ext[1], ext[2]);
-        const BlockShape s = block_shape<kCells>(ex, ey, ez);
+        const BlockShape s = block_shape(ex, ey, ez);
         const bool live = vol != 0.0;
         // positively oriented vertices in the pair's axis order (the face tests need the orientation)
         const bool flip = (vol < 0.0) != swap;
@@ -127,7 +126,7 @@ struct PairLoader {
         double s[4][3];
         for (int q = 0; q < 4; ++q)
             for (int a = 0; a < 3; ++a) s[q][a] = pd.S[3 * q + a];
-        return make_block<kCells>(lo, e, s, unit);
+        return make_block(lo, e, s, unit);
     }
     __device__ __forceinline__ Block block(int2 e) const {
         return block_of(srcs.get(int(unsigned(e.y) >> kUnitBits)).pd[e.x], unsigned(e.y) & kUnitMask);
@@ -160,7 +159,7 @@ struct TileFeed {
     int64_t it = 0, it_end = 0;
     TileHead head;  // of item `it` while it < it_end
 
-    __device__ __forceinline__ bool operator()(Lds& L, int lane) {
+    __device__ __forceinline__ bool operator()(BlockLds& L, int lane) {
         if (it == it_end) {
             unsigned base = 0;
             if (lane == 0) base = atomicAdd(queue_counter, 1u);
@@ -215,9 +214,9 @@ struct TileFeed {
 template <class Sources>
 __device__ __forceinline__ void deposit_tiles(const Sources& srcs, const int2* __restrict__ entries, int64_t n_items, int chunk,
                                               unsigned* __restrict__ queue_counter, unsigned long long* __restrict__ counters) {
-    __shared__ Lds lds[kWaves];
+    __shared__ BlockLds lds[kWaves];
     const int lane = threadIdx.x & 63;
-    Lds& L = lds[threadIdx.x >> 6];
+    BlockLds& L = lds[threadIdx.x >> 6];
     init_wave(L, lane);
     WaveState w;
     TileFeed<Sources> feed{srcs, entries, n_items, chunk, queue_counter, w};

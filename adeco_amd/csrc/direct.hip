@@ -9,7 +9,7 @@
 // nothing but the tets is read from memory.
 // Against the one-tet-per-thread kernel (deposit.hip), whose waves run as long as their largest tet
 // walks its cells: one meta-patch of 2 058 tets on 16^3 cells 104 us against 900-1130, a leaf's 98 784 tets
-// on 16^3 cells 172 against 1420-1530, 196 608 tets on 64^3 cells 0.31 ms against 3.8.  All leaves of an
+// on 16^3 cells 170 against 1420-1530, 196 608 tets on 64^3 cells 0.29 ms against 3.8.  All leaves of an
 // octree in one launch instead of one each: 64 leaves, 1.86 M pairs, 16^3 cells 0.66 ms against 15.2.
 // What bounds it: a small launch lasts as long as one wave's chain of passes (classify, clip, recompute:
 // 20-30 us each, at mostly one wave per SIMD); a large one is bound as the batched form is (blocks.hip).
@@ -31,9 +31,7 @@ namespace {
 
 constexpr int kWaves = 4;
 constexpr int kThreads = 64 * kWaves;
-constexpr int kCells = 16;
-using Lds = BlockLds<kCells>;
-static_assert((sizeof(Lds) * kWaves + 1279) / 1280 * 1280 * 2 <= 160 * 1024, "2 workgroups per CU");
+static_assert((sizeof(BlockLds) * kWaves + 1279) / 1280 * 1280 * 2 <= 160 * 1024, "2 workgroups per CU");
 
 // Tets of one grid.
 struct OneGrid {
@@ -140,7 +138,7 @@ struct DirectLoader {
         V3<double> v[4];
         (void)tets.fetch(e.x, v);
         const TetCover t = cover_of(v, tets.grid(e.x));
-        return make_block<kCells>(t.lo, t.e, t.s, unsigned(e.y) & kUnits);
+        return make_block(t.lo, t.e, t.s, unsigned(e.y) & kUnits);
     }
     __device__ __forceinline__ Place place(int2 e, const int lo[3]) const {
         const GridDesc& g = tets.grid(e.x);
@@ -168,7 +166,7 @@ struct DirectFeed {
 
     // One step: a new item (whose blocks follow at once when no tet has more than one), or the next 64
     // blocks of the current one.
-    __device__ __forceinline__ bool operator()(Lds& L, int lane) {
+    __device__ __forceinline__ bool operator()(BlockLds& L, int lane) {
         const bool fresh = cursor >= total;
         unsigned t;  // this lane's tet, its block below
         bool live;
@@ -209,7 +207,7 @@ struct DirectFeed {
         if (fresh) {
             cnt = 0;
             if (live) {
-                const BlockShape s = block_shape<kCells>(c.e[0], c.e[1], c.e[2]);
+                const BlockShape s = block_shape(c.e[0], c.e[1], c.e[2]);
                 cnt = unsigned(s.n[0]) * unsigned(s.n[1]) * unsigned(s.n[2]);
             }
             cursor = total = 0;
@@ -233,7 +231,7 @@ struct DirectFeed {
                     c.s[0][a] = c.s[3][a];
                     c.s[3][a] = s0;
                 }
-            const Block b = make_block<kCells>(c.lo, c.e, c.s, unit);
+            const Block b = make_block(c.lo, c.e, c.s, unit);
             key = classify_block(b);
             if (key == kBlockTet || key == kBlockFull) {
                 const GridDesc& g = tets.grid(int(t));
@@ -252,9 +250,9 @@ template <class Tets>
 __global__ void __launch_bounds__(kThreads, 2) k_deposit_direct(Tets tets, unsigned n_tets, unsigned per_item, unsigned per_pop,
                                                                 double tet_mass, double* __restrict__ grid,
                                                                 DirectCounters* __restrict__ ctr) {
-    __shared__ Lds lds[kWaves];
+    __shared__ BlockLds lds[kWaves];
     const int lane = threadIdx.x & 63;
-    Lds& L = lds[threadIdx.x >> 6];
+    BlockLds& L = lds[threadIdx.x >> 6];
     init_wave(L, lane);
     WaveState w;
     DirectFeed<Tets> feed{tets, grid, tet_mass, n_tets, per_item, per_pop, &ctr->next, w};

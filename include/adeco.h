@@ -399,7 +399,7 @@ void adeco_selftest_decomposition(int decomposition, int32_t* corners24);
  * was summed from. */
 void adeco_selftest_column_f64(const double* tet12, int ls, int use_signed, double* vol6_out, double* sab_out);
 /* The block form's clip on the host: tet12 in cells from the block's corner, cells3 = the block's
- * cells per axis (at most 16 together); shares_out[(a * cells3[1] + b) * cells3[2] + k] = the share
+ * cells per axis (at most 24 together); shares_out[(a * cells3[1] + b) * cells3[2] + k] = the share
  * of the tet in cell (a, b, k) as the block clip sums it, alone_out = the same cell recomputed alone.
  * Returns the number of cells, or -1. */
 int adeco_selftest_block_f64(const double* tet12, const int* cells3, double* shares_out, double* alone_out);

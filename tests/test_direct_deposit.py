@@ -17,6 +17,21 @@ pytestmark = pytest.mark.gpu
 BOX = np.array([0, 32, 0, 32, 0, 32], np.float32)
 
 
+@pytest.mark.parametrize("extents", [
+    [(1, 1, 24), (2, 2, 6), (1, 4, 6), (2, 3, 4)],   # one block of 24 cells
+    [(1, 1, 25), (1, 2, 13), (2, 2, 7), (3, 3, 3)],  # just over
+])
+@pytest.mark.parametrize("mode", [A.MODE_PLAIN, A.MODE_BATCHED])
+def test_soup_around_the_largest_block(extents, mode):
+    tets = soup_of_extents(np.random.default_rng(11), extents, 80)
+    print(f"[direct] {extents} mode {mode}", flush=True)
+    got = A.deposit_soup(tets, BOX, 32, 1.0, mode=mode, precision=A.PREC_FP64)
+    with O.cell_scaling(O.EXACT):
+        want = O.deposit_soup_ld(tets, BOX, 32, 1.0)
+    assert O.max_rel_err(got, want, tet_mass=1.0) <= 1e-6
+    assert abs(got.sum() - want.sum()) <= 1e-9 * want.sum()
+
+
 @pytest.mark.parametrize("n", [1, 63, 65, 700])
 @pytest.mark.parametrize("extents", [
     [(1, 1, 1), (1, 2, 2)],                          # one block each: taken without a second walk
