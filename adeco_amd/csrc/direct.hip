@@ -268,13 +268,15 @@ hipError_t launch(const Tets& tets, int64_t n_tets, int dims, bool small_tets, d
     if (n_tets <= 0) return hipSuccess;
     int cus = 256;
     (void)hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, device);
-    // tets per item: 64 fill a wave's lanes; fewer where that leaves resident waves without work (a small
-    // launch is over when its slowest wave is, and large tets bring many blocks each): about two items
-    // per resident wave
+    // tets per item: 64 fill a wave's lanes; fewer where that leaves 7 of 8 resident waves without work.  (A small
+    // launch is over when its slowest wave is, so a wave's chain of passes should be short; but passes with
+    // few lanes cost as much as full ones and get in each other's way.  2 058 tets on 16^3 cells, the call: two
+    // items per resident wave 160 us, one for half 120, for a quarter or an eighth 90-100; 98 784 tets: 343, 285,
+    // 282 us; 196 608 tets on 64^3 cells: 457, 445, 440.)
     const int64_t waves = int64_t(cus) * 2 * kWaves;
     // (64 tets of up to 2^26 blocks each would overflow their 32-bit sum on grids beyond 512^3)
     int per_item = dims <= 512 ? 64 : 32;
-    while (per_item > 1 && n_tets < 2 * waves * per_item) per_item >>= 1;
+    while (per_item > 1 && 8 * n_tets < waves * per_item) per_item >>= 1;
     const int64_t items = (n_tets + per_item - 1) / per_item;
     const WaveLaunch w = wave_launch(items, block_occupancy(), kWaves, device);
     // items per pop: one where the tets' blocks may differ much in number (45 M blocks of 6.7 M pairs on 32^3-cell

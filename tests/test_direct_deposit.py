@@ -52,6 +52,17 @@ def test_soup(n, extents):
     assert abs(got.sum() - want.sum()) <= 1e-9 * max(want.sum(), 1.0)
 
 
+@pytest.mark.parametrize("dims", [1, 4, 5, 16])
+def test_batched_soup_on_either_side_of_four_tets_per_cell(dims):
+    tets = soup_of_extents(np.random.default_rng(dims), [(1, 2, 2), (3, 3, 3), (9, 12, 14)], 100)  # 300 >= 4 * 4^3
+    print(f"[direct] batched soup {dims}", flush=True)
+    got = A.deposit_soup(tets, BOX, dims, 1.0, mode=A.MODE_BATCHED)
+    with O.cell_scaling(O.EXACT):
+        want = O.deposit_soup_ld(tets, BOX, dims, 1.0)
+    assert O.max_rel_err(got, want, tet_mass=1.0) <= 1e-6
+    assert abs(got.sum() - want.sum()) <= 1e-9 * want.sum()
+
+
 @pytest.mark.parametrize("dims", [1, 2, 17, 64])
 def test_lattice_tets_all_and_listed(dims):
     rng = np.random.default_rng(dims)
