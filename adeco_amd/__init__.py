@@ -84,7 +84,8 @@ def get_cell_scaling() -> int:
 def set_boundary_form(decomposition=None, tet_mass=None, mode=None, precision=None):
     """Library-wide form of DepositWrapper.deposit_tets (the boundary call): the tets of a cube
     (default DECOMP_REF_EFFECTIVE), the mass of one tet (default 1), the kernel form (default
-    MODE_PLAIN; MODE_BATCHED runs the batched persistent deposit on the patches' tets) and the
+    MODE_PLAIN; MODE_BATCHED runs the batched persistent deposit, from a soup of the patches' tets
+    where they are few per cell) and the
     precision (default PREC_FP64; the other modes need MODE_BATCHED).  Returns the previous form."""
     lib = load()
     prev = {"decomposition": lib.adeco_get_tet_decomposition(), "tet_mass": lib.adeco_get_tet_mass(),
@@ -556,7 +557,7 @@ def get_launch_shape() -> tuple:
 
 def roi_deposit_plain(lattice: ResidentLattice, roi, dims: int, decomposition: int = DECOMP_KUHN,
                       tet_mass: float = 1.0 / 6.0):
-    """The serial baseline of Server: one request, plain one-tet-per-thread kernel, synchronous.
+    """The serial baseline of Server: one request, plain form of the kernel, synchronous.
     Returns the (dims, dims, dims) FP32 density and the number of selected tets."""
     roi = np.ascontiguousarray(roi, np.float64)
     out = np.empty(int(dims) ** 3, np.float32)

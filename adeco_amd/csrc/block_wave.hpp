@@ -43,7 +43,7 @@ struct BlockLds {
 // z up to 6 (more where x and y have few) and y what is left, the cells spread evenly over an axis' blocks.
 // Large blocks cut fewer faces between blocks, and planes across z cost least.  24 cells are what the LDS of a
 // wave holds; against 16 (2 x 2 x 4): 15.3 M pairs on 16^3-cell leaves 4.02 -> 3.71 ms, 6.7 M pairs on
-// 32^3-cell leaves 10.9 -> 9.75, a request of 200^3 cells 515 -> 409 us.
+// 32^3-cell leaves 10.9 -> 9.75, a 64^3 request on a 128^3 lattice 515 -> 409 us.
 struct BlockShape {
     int b[3], n[3];
 };

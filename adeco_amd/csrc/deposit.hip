@@ -4,7 +4,8 @@
 // resample_without_connectivity_GPU, AdDeposit2Grid.cu:139-211, runs one warp per Lagrangian cell
 // and one lane per covered cell).  Here every lane owns one tet end to end: it loads the 4
 // vertices (coalesced SoA loads for the resident lattice), computes the covered range and walks
-// it.  The batched form (batched.hip) is the load-balanced alternative.
+// it.  They serve what the block form does not take: the reference's cell scaling, grids of 1024 cells, and
+// calls that ask for work statistics (direct.hip runs the plain form otherwise).
 #include <hip/hip_runtime.h>
 
 #include "deposit_tet.hpp"

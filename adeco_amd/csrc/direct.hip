@@ -8,8 +8,8 @@
 // and full queues are clipped by the whole wave.  So a wave's lanes share the cells of a large tet, and
 // nothing but the tets is read from memory.
 // Against the one-tet-per-thread kernel (deposit.hip), whose waves run as long as their largest tet
-// walks its cells: one meta-patch of 2 058 tets on 16^3 cells 104 us against 900-1130, a leaf's 98 784 tets
-// on 16^3 cells 170 against 1420-1530, 196 608 tets on 64^3 cells 0.29 ms against 3.8.  All leaves of an
+// walks its cells: one meta-patch of 2 058 tets on 16^3 cells 37 us against 900-1130, a leaf's 98 784 tets
+// on 16^3 cells 115 against 1420-1530, 196 608 tets on 64^3 cells 0.28 ms against 3.8.  All leaves of an
 // octree in one launch instead of one each: 64 leaves, 1.86 M pairs, 16^3 cells 0.66 ms against 15.2.
 // What bounds it: a small launch lasts as long as one wave's chain of passes (classify, clip, recompute:
 // 20-30 us each, at mostly one wave per SIMD); a large one is bound as the batched form is (blocks.hip).

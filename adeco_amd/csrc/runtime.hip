@@ -193,8 +193,8 @@ using namespace adeco;
 namespace {
 
 // One device's share of a boundary call: passes over its patch range within the budget.  The
-// plain form runs one thread per tet over the uploaded patches; the batched form expands each
-// pass's patches into a tet soup on the device and runs the batched persistent deposit on it, so
+// plain form deposits straight from the uploaded patches; the batched form, where a pass has few tets per
+// cell, expands them into a tet soup on the device and runs the batched persistent deposit on it, so
 // a pass budgets the soup and the soup's candidate space as well (the tile map, about one 64th of
 // the candidates in 4 bytes each, is allocated on top).
 adeco_status deposit_patches_on_device(int dev, size_t first_patch, size_t n_patches, const float* positions,
@@ -245,7 +245,7 @@ adeco_status deposit_patches_on_device(int dev, size_t first_patch, size_t n_pat
                            hipMemcpyHostToDevice, ds.stream);
         if (e != hipSuccess) return hip_fail(e, "positions upload");
         // Batched: many small tets (4 or more per cell, the leaf deposit's rule) need no soup, pair lines, scan, tile
-        // map or read-back: 98 784 tets on 16^3 cells, the call 277 -> 228 us
+        // map or read-back: 80 patches on 24^3 cells, the call 277 -> 228 us
         counted = batched && precision == ADECO_PREC_FP64 && direct && np * tets_per_patch >= 4 * ncell;
         if (batched && !counted) {
             e = launch_patches_to_soup(ds.pos.as<float>(), int64_t(np), m, decomp, soup.as<float>(), ds.stream);

@@ -20,8 +20,8 @@
 //     (mass / cell volume, as AdOctreeGridWriter::write_patch) and an event is recorded on the
 //     step stream; a copier thread waits for that event, moves the density to the caller's buffer
 //     and frees the slot.
-// adeco_roi_deposit_plain is the serial baseline: the same selection, then the plain
-// one-tet-per-thread kernel, one request at a time.
+// adeco_roi_deposit_plain is the serial baseline: the same selection, then the plain form (direct.hip), one
+// request at a time.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>

@@ -60,11 +60,10 @@ TET_MASS = 1.0 / 6.0
 FP64_PEAK_TFLOPS = 78.6  # MI355X FP64 vector peak (the roof of an FP64 VALU-bound kernel)
 FP32_PEAK_TFLOPS = 157.3  # MI355X FP32 vector peak (packed)
 HBM_PEAK_GBS = 8000.0
-# HBM bytes per launch of k_deposit_waves<FP64, false> at 16^3-cell leaves: rocprofv3 FETCH_SIZE
-# and WRITE_SIZE (KiB per dispatch) scaled by what each reads for a 1 GiB copy (2.0 and 1.0),
-# profiles/deposit_waves_c3_pmc.md (256^3 infall workload) and profiles/deposit_waves_c2_pmc.md
-# (128^3)
-TRAFFIC_BYTES = {"c3": 22706736.9375 * 2 * 1024 + 18270762.125 * 1024, "c2": 2575602.0 * 2 * 1024 + 1951831.875 * 1024}
+# HBM bytes per launch of the FP64 leaf deposit (k_deposit_direct) at 16^3-cell leaves: rocprofv3
+# FETCH_SIZE and WRITE_SIZE (KiB per dispatch) scaled by what each reads for a 1 GiB copy (2.0 and
+# 1.0), profiles/deposit_blocks.md (256^3 infall workload and 128^3)
+TRAFFIC_BYTES = {"c3": 5919428.9375 * 2 * 1024 + 19562973.875 * 1024, "c2": 528110.8125 * 2 * 1024 + 2061348.8125 * 1024}
 
 
 def log(*a):
@@ -248,7 +247,7 @@ def roofline_of(work, dims, kernel_ms, lat, n_leaves, counts=None, levels=None, 
            "achieved": achieved, "peak": FP64_PEAK_TFLOPS, "unit": "TFLOP/s", "frac": achieved / FP64_PEAK_TFLOPS,
            "frac_of_fp32_peak": achieved / FP32_PEAK_TFLOPS, "traffic": traffic,
            "flops_per_launch": w["flops"], "flops_rel_std_err": w["flops_rel_std_err"], "kernel_ms": kernel_ms,
-           "kernel": "k_deposit_waves<FP64>", "leaf_dims": dims}
+           "kernel": "FP64 block deposit (k_deposit_direct, k_deposit_blocks)", "leaf_dims": dims}
     if alg_bytes is not None:
         rec.update({"algorithmic_bytes": alg_bytes, "nonzero_contributions": nonzero,
                     "hbm_achieved_gbs": alg_bytes / (kernel_ms * 1e-3) / 1e9,
@@ -360,7 +359,7 @@ def serve_study(rates, count, seed=5, max_inflight=16):
                    "plain_serial_makespan_s": finish, "batched_vs_plain_max_rel_err": err, "by_resolution": by_res}
             if serve_flops is not None:
                 ach = serve_flops / float(st["step_kernel_s"]) / 1e12
-                rec["roofline"] = {"bound": "valu", "kernel": "k_deposit_step<FP64>", "achieved": ach,
+                rec["roofline"] = {"bound": "valu", "kernel": "k_step_blocks", "achieved": ach,
                                    "peak": FP64_PEAK_TFLOPS, "unit": "TFLOP/s", "frac": ach / FP64_PEAK_TFLOPS,
                                    "flops": serve_flops, "kernel_s": float(st["step_kernel_s"])}
             log(f"[serve] {rate:g} req/s: batched p50 {p50 * 1e3:.1f} ms p99 {p99 * 1e3:.1f} ms "
@@ -603,8 +602,7 @@ def boundary_study(reps=2):
     workload, called as the reference's worker calls it (AdDynamicLoadBalancing.h:200-205): once
     per octree leaf, with the leaf's gathered meta-patches in host memory (its meta-cell list, the
     reference's gather order), the leaf's float box, 16^3 cells, the reference's tets of mass 1,
-    into a zeroed float grid.  The plain form (one thread per tet, the reference kernel's
-    structure) against the batched form; host-to-device copies of the patches and the grid
+    into a zeroed float grid.  The plain form (straight from the patches) against the batched form; host-to-device copies of the patches and the grid
     readback are inside the timed loop."""
     from adeco_amd.lattice import meta_patches
     lat = make_lattice(N, RMS, seed=SEED)

@@ -50,7 +50,7 @@ typedef int adeco_status;
 #define ADECO_DECOMP_KUHN 2          /* six tets around the (0,0,0)-(1,1,1) diagonal */
 
 /* Deposit execution forms. */
-#define ADECO_MODE_PLAIN 0   /* one tet per thread, one launch per output grid */
+#define ADECO_MODE_PLAIN 0   /* straight from the tets, nothing prepared (boundary: one launch per grid) */
 #define ADECO_MODE_BATCHED 1 /* persistent work-queue launch over all grids, load-balanced (tet, cell) work */
 
 /* Precision of the clip (accumulation is always FP64 on the device). */
@@ -70,8 +70,8 @@ const char* adeco_last_error(void);
 /* Library-wide form of the boundary call adeco_deposit_patches (set before concurrent use): the 6
  * tets of a lattice cube (default ADECO_DECOMP_REF_EFFECTIVE, the reference's), the mass of one tet
  * (default 1, as resample_meta_patch, AdDepositTets2Grid.h:1007-1053), the kernel form (default
- * ADECO_MODE_PLAIN, one thread per tet like the reference's kernel; ADECO_MODE_BATCHED expands
- * each pass's patches into a tet soup on the device and runs the batched persistent deposit on it)
+ * ADECO_MODE_PLAIN, straight from the patches; ADECO_MODE_BATCHED deposits passes of few tets per
+ * cell from a tet soup expanded on the device, and reports counts of blocks and recomputes)
  * and the precision (default ADECO_PREC_FP64; MIXED and FP32 need the batched form). */
 adeco_status adeco_set_tet_decomposition(int decomposition);
 int adeco_get_tet_decomposition(void);
@@ -153,7 +153,7 @@ adeco_status adeco_lattice_deposit_grid(adeco_lattice lat, int decomposition, do
                                         uint64_t* stats);
 
 /* Deposits a tet soup (float [n][4][3]) onto one grid (precision study inputs).  MODE_PLAIN runs
- * the one-tet-per-thread FP64 kernel; MODE_BATCHED the persistent (tet, cell) kernel in the given
+ * the plain FP64 form (with stats, the one-tet-per-thread kernel); MODE_BATCHED the persistent kernel in the given
  * precision, with its kernel time, partial cells and FP64 recomputes in adeco_last_timings. */
 adeco_status adeco_deposit_soup(int device_id, const float* tets, int64_t n_tets, const float* bbox6,
                                 int dims, double tet_mass, int mode, int precision, double* grid_out,
@@ -380,8 +380,8 @@ adeco_status adeco_serve_wait(adeco_server srv, uint64_t request_id, double time
 adeco_status adeco_serve_stats_get(adeco_server srv, adeco_serve_stats* out);
 /* Finishes every queued request, then stops the threads and frees the device buffers. */
 adeco_status adeco_serve_destroy(adeco_server srv);
-/* The serial baseline: the same selection and output for one box, deposited by the plain
- * one-tet-per-thread kernel, synchronously.  n_tets_out (nullable) receives the selected tets. */
+/* The serial baseline: the same selection and output for one box, deposited by the
+ * plain form of the kernel, synchronously.  n_tets_out (nullable) receives the selected tets. */
 adeco_status adeco_roi_deposit_plain(adeco_lattice lat, int decomposition, double tet_mass, const double* roi6,
                                      int dims, float* density_out, int64_t* n_tets_out);
 
