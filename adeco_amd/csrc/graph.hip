@@ -11,7 +11,8 @@
 //     replay that needs more sets an overflow flag, deposits nothing and reports ADECO_EOVERFLOW.
 // Either graph owns every buffer its kernels write (binning counters, pair lists, leaf geometry,
 // pair data, tile map, leaf grids, counters) and its own copies of the octree tables the binning
-// reads, so deposits through the octree handle cannot move them; the lattice must outlive it.
+// reads, so deposits through the octree handle cannot move them and destroying it takes nothing away; the
+// lattice must outlive it.
 #include <hip/hip_runtime.h>
 
 #include "../../include/adeco.h"
@@ -26,7 +27,7 @@ using namespace adeco;
 static size_t align_up(size_t b) { return (b + 255) & ~size_t(255); }
 
 struct adeco_deposit_graph_s {
-    adeco_octree_s* T = nullptr;
+    DeviceState* ds = nullptr;  // of the lattice's device (the octree may be gone before the graph)
     int device = 0, dims = 0, precision = 0;
     int64_t n_leaves = 0;
     DevBuf geom, work, tiles, grids, counters;
@@ -64,7 +65,7 @@ adeco_status adeco_deposit_graph_create(adeco_octree T, int dims, int decomposit
     adeco_status st;
     if (T->binned_decomposition != decomposition && (st = octree_bin_tets(T, decomposition))) return st;
     auto* G = new adeco_deposit_graph_s();
-    G->T = T;
+    G->ds = &ds;
     G->device = T->L->device;
     G->dims = dims;
     G->precision = precision;
@@ -146,7 +147,7 @@ adeco_status adeco_deposit_graph_create_step(adeco_octree T, int dims, int decom
     // one eager binning and candidate space: the capacities, and the octree's tables
     if ((st = octree_bin_tets(T, decomposition))) return st;
     auto* G = new adeco_deposit_graph_s();
-    G->T = T;
+    G->ds = &ds;
     G->device = T->L->device;
     G->dims = dims;
     G->precision = precision;
@@ -265,7 +266,7 @@ adeco_status adeco_deposit_graph_grids(adeco_deposit_graph G, int64_t first_leaf
     const int64_t cells = int64_t(G->dims) * G->dims * G->dims;
     hipError_t e = hipSetDevice(G->device);
     if (e == hipSuccess)
-        e = download(*G->T->L->ds, G->stream, out, G->grids.as<double>() + first_leaf * cells, size_t(n_leaves * cells) * 8);
+        e = download(*G->ds, G->stream, out, G->grids.as<double>() + first_leaf * cells, size_t(n_leaves * cells) * 8);
     return e == hipSuccess ? ADECO_OK : hip_fail(e, "deposit graph grids");
 }
 
