@@ -88,7 +88,7 @@ __global__ void __launch_bounds__(256) k_block_setup(LatticeView lat, PackedCorn
         const int ax = role_axis(code, 0), ay = role_axis(code, 1), za = code & 3;
         const int ex = pick(ax, ext[0], ext[1], ext[2]), ey = pick(ay, ext[0], ext[1], ext[2]), ez = pick(za, ext[0], ext[1], ext[2]);
         const BlockShape s = block_shape(ex, ey, ez);
-        const bool live = vol != 0.0;
+        const bool live = has_volume(vol);
         // positively oriented vertices in the pair's axis order (the face tests need the orientation)
         const bool flip = (vol < 0.0) != swap;
         unsigned long long* o = rows + threadIdx.x * (kWords + 1);

@@ -99,6 +99,11 @@ ADECO_HD void deposit_tet_f64(const V3<double> v[4], const GridGeom& g, double t
     }
 }
 
+// Whether a tet of this volume (or 6 times it) deposits: none without volume, and none with a vertex that is not
+// finite, whose volume is not finite either (every coordinate is a factor of it; finite floats don't overflow).
+// The routine above drops the latter cell by cell, where NaN and infinite volumes fail its tests.
+ADECO_HD bool has_volume(double vol) { return fabs(vol) > 0.0 && fabs(vol) <= 1.7976931348623157e308; }
+
 ADECO_HD bool is_sentinel(float x, float y, float z) {  // AdDepositTets2Grid.h:1029-1038
     const float s = fabsf(x - 666.f) + fabsf(y - 666.f) + fabsf(z - 666.f);
     return double(s) < 1.E-03;

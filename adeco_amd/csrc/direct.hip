@@ -184,7 +184,7 @@ struct DirectFeed {
             next += per_item;
             t = first + unsigned(lane);
             live = unsigned(lane) < per_item && t < end;
-            n_units += __popcll(__ballot(live));  // (a tet without volume counts as one block)
+            n_units += __popcll(__ballot(live));  // (a tet that deposits nothing counts as one block)
         } else {
             const int item = item_of_unit(L, lane, start, cnt, cursor);
             const unsigned item_start = unsigned(__shfl(int(start), max(item, 0), 64));
@@ -202,7 +202,7 @@ struct DirectFeed {
             c = cover_of(v, tets.grid(int(t)));
             code = c.code;
             vol = vol6(v[0], v[1], v[2], v[3]);
-            live = live && vol != 0.0;
+            live = live && has_volume(vol);
         }
         if (fresh) {
             cnt = 0;
