@@ -154,6 +154,32 @@ ADECO_HD float qdiv(float a, float b) {
 #endif
 }
 
+// n / d for n < 2^30 and 1 <= d < 2^30 without the integer division sequence: the FP64 reciprocal
+// refined once is accurate to ~2^-50, so the truncated product is the quotient or one less (exact
+// multiples), fixed by one integer correction each way
+ADECO_HD unsigned udiv_small(unsigned n, unsigned d) {
+#if defined(__HIP_DEVICE_COMPILE__)
+    const double dd = double(d);
+    double r = __builtin_amdgcn_rcp(dd);
+    r = fma(fma(-dd, r, 1.0), r, r);
+    unsigned q = unsigned(double(n) * r);
+    q -= unsigned(q * d > n);
+    q += unsigned((q + 1) * d <= n);
+    return q;
+#else
+    return n / d;
+#endif
+}
+
+// 1 / v to a few ulps of a float
+ADECO_HD float rcp_approx(float v) {
+#if defined(__HIP_DEVICE_COMPILE__)
+    return __builtin_amdgcn_rcpf(v);
+#else
+    return 1.0f / v;
+#endif
+}
+
 // Fraction of a tet's volume on the far side (d > 0) of a plane, from the 4 vertex distances.
 // With a = the beyond magnitudes, c = the near ones (|d|), and D = the product over the vertex
 // pairs on opposite sides of (|d_i| + |d_j|) (= |d_i - d_j|, no cancellation):

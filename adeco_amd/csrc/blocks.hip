@@ -73,36 +73,16 @@ __global__ void __launch_bounds__(256) k_block_setup(LatticeView lat, PackedCorn
         lattice_tet_vertices(lat, ct, pairs[p], v);
         const GridDesc& g = grids[gi];
         const double vol = vol6(v[0], v[1], v[2], v[3]) / 6.0;
-        // vertices in cells
-        double c[4][3];
-        int lo[3], ext[3];
-        for (int a = 0; a < 3; ++a) {
-            for (int q = 0; q < 4; ++q) c[q][a] = g.scale[a] * (comp(v[q], a) - g.gmin[a]);
-            int h;
-            covered(fmin(fmin(c[0][a], c[1][a]), fmin(c[2][a], c[3][a])), fmax(fmax(c[0][a], c[1][a]), fmax(c[2][a], c[3][a])), g.dims,
-                    lo[a], h);
-            ext[a] = h - lo[a] + 1;
-        }
-        const int code = role_code(ext);
-        const bool swap = code & 4;
-        const int ax = role_axis(code, 0), ay = role_axis(code, 1), za = code & 3;
-        const int ex = pick(ax, ext[0], ext[1], ext[2]), ey = pick(ay, ext[0], ext[1], ext[2]), ez = pick(za, ext[0], ext[1], ext[2]);
-        const BlockShape s = block_shape(ex, ey, ez);
+        TetCover t = cover_of(v, g);
+        const BlockShape s = block_shape(t.e[0], t.e[1], t.e[2]);
         const bool live = has_volume(vol);
-        // positively oriented vertices in the pair's axis order (the face tests need the orientation)
-        const bool flip = (vol < 0.0) != swap;
+        orient(t, vol);
         unsigned long long* o = rows + threadIdx.x * (kWords + 1);
-        for (int q = 0; q < 4; ++q) {
-            const int at = flip && (q == 0 || q == 3) ? 3 - q : q;
-            o[3 * at] = __double_as_longlong(pick(ax, c[q][0], c[q][1], c[q][2]));
-            o[3 * at + 1] = __double_as_longlong(pick(ay, c[q][0], c[q][1], c[q][2]));
-            o[3 * at + 2] = __double_as_longlong(pick(za, c[q][0], c[q][1], c[q][2]));
-        }
+        for (int q = 0; q < 4; ++q)
+            for (int r = 0; r < 3; ++r) o[3 * q + r] = __double_as_longlong(t.s[q][r]);
         o[12] = __double_as_longlong(live ? tet_mass * (g.cell_vol / fabs(vol)) : 0.0);
-        unsigned long long pack = (unsigned long long)code << 60;
-        pack |= (unsigned long long)pick(ax, lo[0], lo[1], lo[2]) | (unsigned long long)ex << 30;
-        pack |= (unsigned long long)pick(ay, lo[0], lo[1], lo[2]) << 10 | (unsigned long long)ey << 40;
-        pack |= (unsigned long long)pick(za, lo[0], lo[1], lo[2]) << 20 | (unsigned long long)ez << 50;
+        unsigned long long pack = (unsigned long long)t.code << 60;
+        for (int r = 0; r < 3; ++r) pack |= (unsigned long long)t.lo[r] << (10 * r) | (unsigned long long)t.e[r] << (30 + 10 * r);
         o[13] = live ? pack : 0ull;  // extent 0 marks a dead pair
         o[14] = (unsigned long long)unsigned(gi);
         o[15] = 0ull;
@@ -243,7 +223,7 @@ __global__ void __launch_bounds__(kThreads, 2) k_step_blocks(const TileSource* _
     deposit_tiles(ManySources{sources}, entries, n_entries, chunk, queue_counter, counters);
 }
 
-// This tet's shares on the host (the same code; tests only).
+// Shares summed on the host as the lanes of a wave do (the same code; tests only).
 struct HostShares {
     double* a;
     static double term(double share) { return share; }
@@ -315,4 +295,50 @@ extern "C" int adeco_selftest_block_f64(const double* t, const int* cells3, doub
         alone[i] = exact_cell_share(lx, ly, lz, [&](int j) -> double& { return keep[j]; });
     }
     return n;
+}
+
+// The block deposit of a tet soup on the host, block by block (the same code; tests only).
+extern "C" int adeco_selftest_deposit_blocks_f64(const float* tets, int64_t n_tets, const float* bbox6, int dims, double tet_mass,
+                                                 double* grid_out, int64_t* recomputes_out) {
+    using namespace adeco;
+    if (!tets || n_tets < 0 || !bbox6 || dims < 1 || dims > 1023 || !grid_out) return ADECO_EINVAL;
+    const GridDesc g = make_grid_desc(make_grid_geom(bbox6, dims), 0);
+    int64_t recomputes = 0;
+    for (int64_t i = 0; i < n_tets; ++i) {
+        V3<double> v[4];
+        for (int q = 0; q < 4; ++q) v[q] = mk(double(tets[12 * i + 3 * q]), double(tets[12 * i + 3 * q + 1]), double(tets[12 * i + 3 * q + 2]));
+        const double vol = vol6(v[0], v[1], v[2], v[3]);
+        if (!has_volume(vol)) continue;
+        TetCover t = cover_of(v, g);
+        orient(t, vol);
+        const BlockShape s = block_shape(t.e[0], t.e[1], t.e[2]);
+        for (unsigned u = 0; u < unsigned(s.n[0] * s.n[1] * s.n[2]); ++u) {
+            const Block b = make_block(t.lo, t.e, t.s, u);
+            const int key = classify_block(b);
+            if (key == kBlockEmpty) continue;
+            const Place p = place_of(b.lo, t.code, dims);
+            if (key < 0) {
+                const double m = key == kBlockTet ? tet_mass : tet_mass * (g.cell_vol / fabs(vol / 6.0));
+                for_cells(b.c, p, [&](int, int64_t at) { grid_out[at] += m; });
+                continue;
+            }
+            double sum[kBlockCells] = {};
+            HostShares shares{sum};
+            LeafSums<HostShares> leaves{shares};
+            block_shares(true, b.x, b.y, b.z, b.c[0], b.c[1], b.c[2], leaves);
+            for_cells(b.c, p, [&](int k, int64_t at) {
+                double f = sum[k];
+                if (f < kSmallShare) {
+                    if (fabs(f) < kNoShare) return;
+                    double keep[15];
+                    const Block cell = cell_of(b, k);
+                    f = exact_cell_share(cell.x, cell.y, cell.z, [&](int j) -> double& { return keep[j]; });
+                    ++recomputes;
+                }
+                if (f > 0.0) grid_out[at] += tet_mass * f;
+            });
+        }
+    }
+    if (recomputes_out) *recomputes_out = recomputes;
+    return ADECO_OK;
 }

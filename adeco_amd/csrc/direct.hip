@@ -101,33 +101,6 @@ struct PatchTets : OneGrid {
     }
 };
 
-// A tet in the cells of a grid: its cover and its vertices, in the cover's axis order.
-struct TetCover {
-    int lo[3], e[3], code;
-    double s[4][3];
-};
-
-__device__ __forceinline__ TetCover cover_of(const V3<double> v[4], const GridDesc& g) {
-    double c[4][3];
-    int lo[3], e[3];
-    for (int a = 0; a < 3; ++a) {
-        for (int q = 0; q < 4; ++q) c[q][a] = g.scale[a] * (comp(v[q], a) - g.gmin[a]);
-        int h;
-        covered(fmin(fmin(c[0][a], c[1][a]), fmin(c[2][a], c[3][a])), fmax(fmax(c[0][a], c[1][a]), fmax(c[2][a], c[3][a])), g.dims,
-                lo[a], h);
-        e[a] = h - lo[a] + 1;
-    }
-    TetCover t;
-    t.code = role_code(e);
-    for (int r = 0; r < 3; ++r) {
-        const int a = role_axis(t.code, r);
-        t.lo[r] = pick(a, lo[0], lo[1], lo[2]);
-        t.e[r] = pick(a, e[0], e[1], e[2]);
-        for (int q = 0; q < 4; ++q) t.s[q][r] = pick(a, c[q][0], c[q][1], c[q][2]);
-    }
-    return t;
-}
-
 // An entry is the tet's index in the launch and the block's index in the tet.
 template <class Tets>
 struct DirectLoader {
@@ -224,13 +197,7 @@ struct DirectFeed {
             }
         }
         if (live) {
-            // positively oriented in the cover's axis order (the face tests need it)
-            if ((vol < 0.0) != bool(code & 4))
-                for (int a = 0; a < 3; ++a) {
-                    const double s0 = c.s[0][a];
-                    c.s[0][a] = c.s[3][a];
-                    c.s[3][a] = s0;
-                }
+            orient(c, vol);
             const Block b = make_block(c.lo, c.e, c.s, unit);
             key = classify_block(b);
             if (key == kBlockTet || key == kBlockFull) {

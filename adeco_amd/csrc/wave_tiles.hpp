@@ -20,19 +20,6 @@ __device__ __forceinline__ int upper_bound_i64(const int64_t* a, int n, int64_t 
     return lo;
 }
 
-// n / d for n < 2^30 and 1 <= d < 2^30 without the integer division sequence: the FP64 reciprocal
-// refined once is accurate to ~2^-50, so the truncated product is the quotient or one less (exact
-// multiples), fixed by one integer correction each way
-__device__ __forceinline__ unsigned udiv_small(unsigned n, unsigned d) {
-    const double dd = double(d);
-    double r = __builtin_amdgcn_rcp(dd);
-    r = fma(fma(-dd, r, 1.0), r, r);
-    unsigned q = unsigned(double(n) * r);
-    q -= unsigned(q * d > n);
-    q += unsigned((q + 1) * d <= n);
-    return q;
-}
-
 __device__ __forceinline__ void wave_sync() {
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
     __builtin_amdgcn_wave_barrier();

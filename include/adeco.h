@@ -403,6 +403,10 @@ void adeco_selftest_column_f64(const double* tet12, int ls, int use_signed, doub
  * of the tet in cell (a, b, k) as the block clip sums it, alone_out = the same cell recomputed alone.
  * Returns the number of cells, or -1. */
 int adeco_selftest_block_f64(const double* tet12, const int* cells3, double* shares_out, double* alone_out);
+/* The block deposit of a tet soup (float [n][4][3]) onto a zeroed grid run on the host, block by block;
+ * recomputes_out (nullable) = the cells recomputed alone.  dims <= 1023. */
+int adeco_selftest_deposit_blocks_f64(const float* tets, int64_t n_tets, const float* bbox6, int dims, double tet_mass,
+                                      double* grid_out, int64_t* recomputes_out);
 /* The DARK_SKY id decoding the reader's kernel uses: lattice site (x, y, z) of an id. */
 void adeco_selftest_dark_sky_site(long long id, int* site3);
 /* The kernels' per-tet FP64 deposit routine run on the host over a tet soup (float [n][4][3]),
