@@ -44,7 +44,8 @@ int deposit_form(int precision, const GridDesc* grids, int64_t n);
 
 // Everything the deposit needs about one binned (grid, tet) pair, written once by the pair setup:
 // one 128-byte line per pair.  In the block form the vertices and the range are in the pair's own axis
-// order (x, y, z: from the shortest to the longest covered extent), bits 60-62 of the range.
+// order (x, y, z: from the shortest to the longest covered extent), bits 60-62 of the range, and mcell is without
+// tet_mass.
 struct alignas(128) PairData {
     double S[12];              // scale_a * (v_q - gmin_a), vertices in the oriented order
     double mcell;              // tet_mass * cell_vol / |V|

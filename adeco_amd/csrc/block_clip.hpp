@@ -24,10 +24,17 @@ namespace adeco {
 
 // Largest number of cells in a block.
 constexpr int kBlockCells = 24;
-// Shares of a cell below kNoShare (18 ulps of the tet: the differences' rounding) are empty; between
-// that and kSmallShare they are recomputed by exact_cell_share.
+// Shares of a cell below kNoShare (18 ulps of the tet, which large tets are first made smaller for: the differences'
+// rounding) are empty; between that and kSmallShare they are recomputed by exact_cell_share.
 constexpr double kNoShare = 4e-15;
 constexpr double kSmallShare = 1e-8;
+// A share this close to a whole cell's is one: a cell that lies wholly in the tet is exact.
+constexpr double kNearFull = 2e-15;
+// Tets of more than 30 cells' volume are replaced by smaller ones, block by block (shrink_tet).
+constexpr double kLargeTet = 1.0 / 30.0;
+// Where more than 20 000 cells' volume are left of one (two faces at a small angle across the block), or where the
+// rounding of its planes' distance counts (tets about 1000 cells wide), the block's cells are recomputed alone.
+constexpr double kHugeTet = 1.0 / 20000.0, kVastTet = 1e-8;
 
 // 1 / b for a positive denominator, within an ulp or two
 ADECO_HD double recip(double b) {

@@ -129,13 +129,15 @@ __device__ __forceinline__ unsigned clip_blocks(const Loader& ld, bool on, int2 
     unsigned long long* sum = &L.sum[0][lane];
     for (int i = 0; i < kBlockCells; ++i) sum[i * kWaveTile] = 0ull;
     LeafQueue leaves{L, lane};
-    block_shares(on, b.x, b.y, b.z, b.c[0], b.c[1], b.c[2], leaves);
+    const bool huge = b.full < kHugeTet;
+    block_shares(on && !huge, b.x, b.y, b.z, b.c[0], b.c[1], b.c[2], leaves);
     leaves.sum(leaves.n);
     unsigned redo = 0u;
     if (!on) return redo;
+    if (huge) return (1u << (b.c[0] * b.c[1] * b.c[2])) - 1u;
     for_cells(b.c, ld.place(e, b.lo), [&](int i, int64_t at) {
         const double f = LaneShares::value(sum[i * kWaveTile]);
-        if (f >= kSmallShare) ld.add(e, at, f);
+        if (f >= kSmallShare) ld.add(e, at, (fabs(f - b.full) <= kNearFull ? b.full : f) * b.scale);
         else if (fabs(f) >= kNoShare) redo |= 1u << i;
     });
     return redo;
@@ -147,7 +149,7 @@ template <class Loader>
 __device__ __forceinline__ void clip_cell(const Loader& ld, int2 e, Block b, int cell, int first, int stride, double* keep) {
     b = cell_of(b, cell);
     const double f = exact_cell_share(b.x, b.y, b.z, [&](int i) -> double& { return keep[i * kWaveTile]; }, first, stride);
-    if (f > 0.0) ld.add(e, ld.place(e, b.lo).corner, f);
+    if (f > 0.0) ld.add(e, ld.place(e, b.lo).corner, f * b.scale);
 }
 
 // A wavefront's state between calls of run_wave.

@@ -80,7 +80,7 @@ __global__ void __launch_bounds__(256) k_block_setup(LatticeView lat, PackedCorn
         unsigned long long* o = rows + threadIdx.x * (kWords + 1);
         for (int q = 0; q < 4; ++q)
             for (int r = 0; r < 3; ++r) o[3 * q + r] = __double_as_longlong(t.s[q][r]);
-        o[12] = __double_as_longlong(live ? tet_mass * (g.cell_vol / fabs(vol)) : 0.0);
+        o[12] = __double_as_longlong(live ? g.cell_vol / fabs(vol) : 0.0);
         unsigned long long pack = (unsigned long long)t.code << 60;
         for (int r = 0; r < 3; ++r) pack |= (unsigned long long)t.lo[r] << (10 * r) | (unsigned long long)t.e[r] << (30 + 10 * r);
         o[13] = live ? pack : 0ull;  // extent 0 marks a dead pair
@@ -106,10 +106,12 @@ struct PairLoader {
         double s[4][3];
         for (int q = 0; q < 4; ++q)
             for (int a = 0; a < 3; ++a) s[q][a] = pd.S[3 * q + a];
-        return make_block(lo, e, s, unit);
+        return make_block(lo, e, s, pd.mcell, unit);
     }
     __device__ __forceinline__ Block block(int2 e) const {
-        return block_of(srcs.get(int(unsigned(e.y) >> kUnitBits)).pd[e.x], unsigned(e.y) & kUnitMask);
+        Block b = block_of(srcs.get(int(unsigned(e.y) >> kUnitBits)).pd[e.x], unsigned(e.y) & kUnitMask);
+        shrink_tet(b);
+        return b;
     }
     __device__ __forceinline__ Place place(int2 e, const int lo[3]) const {
         const TileSource& src = srcs.get(int(unsigned(e.y) >> kUnitBits));
@@ -178,7 +180,7 @@ struct TileFeed {
                 key = classify_block(b);
                 if (key == kBlockTet || key == kBlockFull) {
                     const GridDesc& g = src.grids[pd.grid];
-                    const double m = key == kBlockTet ? src.tet_mass : pd.mcell;
+                    const double m = key == kBlockTet ? src.tet_mass : src.tet_mass * b.full;
                     double* grid = src.grid_buf + g.base;
                     for_cells(b.c, place_of(b.lo, int(pd.range >> 60) & 7, g.dims), [&](int, int64_t at) { unsafeAtomicAdd(grid + at, m); });
                 }
@@ -311,31 +313,33 @@ extern "C" int adeco_selftest_deposit_blocks_f64(const float* tets, int64_t n_te
         if (!has_volume(vol)) continue;
         TetCover t = cover_of(v, g);
         orient(t, vol);
+        const double full = g.cell_vol / fabs(vol / 6.0);
         const BlockShape s = block_shape(t.e[0], t.e[1], t.e[2]);
         for (unsigned u = 0; u < unsigned(s.n[0] * s.n[1] * s.n[2]); ++u) {
-            const Block b = make_block(t.lo, t.e, t.s, u);
+            Block b = make_block(t.lo, t.e, t.s, full, u);
             const int key = classify_block(b);
             if (key == kBlockEmpty) continue;
             const Place p = place_of(b.lo, t.code, dims);
             if (key < 0) {
-                const double m = key == kBlockTet ? tet_mass : tet_mass * (g.cell_vol / fabs(vol / 6.0));
+                const double m = key == kBlockTet ? tet_mass : tet_mass * full;
                 for_cells(b.c, p, [&](int, int64_t at) { grid_out[at] += m; });
                 continue;
             }
+            shrink_tet(b);
             double sum[kBlockCells] = {};
             HostShares shares{sum};
             LeafSums<HostShares> leaves{shares};
-            block_shares(true, b.x, b.y, b.z, b.c[0], b.c[1], b.c[2], leaves);
-            for_cells(b.c, p, [&](int k, int64_t at) {
-                double f = sum[k];
-                if (f < kSmallShare) {
-                    if (fabs(f) < kNoShare) return;
-                    double keep[15];
-                    const Block cell = cell_of(b, k);
+            const bool huge = b.full < kHugeTet;
+            block_shares(!huge, b.x, b.y, b.z, b.c[0], b.c[1], b.c[2], leaves);
+            for_cells(b.c, p, [&](int c, int64_t at) {
+                double f = fabs(sum[c] - b.full) <= kNearFull ? b.full : sum[c], keep[15];
+                if (f < kSmallShare || huge) {
+                    if (fabs(f) < kNoShare && !huge) return;
+                    const Block cell = cell_of(b, c);
                     f = exact_cell_share(cell.x, cell.y, cell.z, [&](int j) -> double& { return keep[j]; });
                     ++recomputes;
                 }
-                if (f > 0.0) grid_out[at] += tet_mass * f;
+                if (f > 0.0) grid_out[at] += tet_mass * f * b.scale;
             });
         }
     }

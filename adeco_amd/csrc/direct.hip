@@ -110,8 +110,13 @@ struct DirectLoader {
     __device__ __forceinline__ Block block(int2 e) const {
         V3<double> v[4];
         (void)tets.fetch(e.x, v);
-        const TetCover t = cover_of(v, tets.grid(e.x));
-        return make_block(t.lo, t.e, t.s, unsigned(e.y) & kUnits);
+        const GridDesc& g = tets.grid(e.x);
+        TetCover t = cover_of(v, g);
+        const double vol = vol6(v[0], v[1], v[2], v[3]);
+        orient(t, vol);
+        Block b = make_block(t.lo, t.e, t.s, qdiv(6.0 * g.cell_vol, fabs(vol)), unsigned(e.y) & kUnits);
+        shrink_tet(b);
+        return b;
     }
     __device__ __forceinline__ Place place(int2 e, const int lo[3]) const {
         const GridDesc& g = tets.grid(e.x);
@@ -198,7 +203,7 @@ struct DirectFeed {
         }
         if (live) {
             orient(c, vol);
-            const Block b = make_block(c.lo, c.e, c.s, unit);
+            const Block b = make_block(c.lo, c.e, c.s, 1.0, unit);
             key = classify_block(b);
             if (key == kBlockTet || key == kBlockFull) {
                 const GridDesc& g = tets.grid(int(t));

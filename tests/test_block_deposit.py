@@ -46,3 +46,76 @@ def test_soups_of_all_block_shapes(extents):
     tets = soup_of_extents(np.random.default_rng(21), extents, 30)
     got, _ = blocks(tets, unit_box(32), 32)
     assert np.abs(got - oracle(tets, unit_box(32), 32)).max() <= 2e-14 * len(tets)
+
+
+def wide_tets(width, seed):
+    """Kuhn tets of 2^3 displaced cubes, each cube `width` cells wide, around the middle of a 32^3 grid."""
+    rng = np.random.default_rng(seed)
+    v = np.stack(np.meshgrid(*[np.arange(3.0)] * 3, indexing="ij"), -1)
+    v = (v + rng.normal(0, 0.2, v.shape) - 1.0) * width + 16.0
+    out = []
+    for p in KUHN:
+        o, vs = np.zeros(3, int), []
+        for s in range(4):
+            vs.append(v[o[0]:o[0] + 2, o[1]:o[1] + 2, o[2]:o[2] + 2].reshape(-1, 3))
+            if s < 3:
+                o[p[s]] += 1
+        out.append(np.stack(vs, 1))
+    return np.concatenate(out).astype(np.float32)
+
+
+def wedges(rng, n, length):
+    """Tets `length` cells long and about a cell thick: faces at small angles across the grid."""
+    t = rng.normal(0, length, (n, 4, 3))
+    axis = rng.integers(0, 3, n)
+    t[np.arange(n), :, axis] = rng.uniform(-1.5, 1.5, (n, 4))
+    return (t + 16.0).astype(np.float32)
+
+
+def rms(a, want):
+    return float(np.sqrt(((a - want) ** 2).sum() / (want ** 2).sum()))
+
+
+WIDE = [("cubes", 27), ("cubes", 80), ("cubes", 120), ("cubes", 400), ("cubes", 1000), ("wedges", 40), ("wedges", 600)]
+
+
+def wide(kind, width):
+    if kind == "cubes":
+        return wide_tets(width, 7)
+    return np.concatenate([wedges(np.random.default_rng(8), 30, width), wide_tets(width, 9)])
+
+
+@pytest.mark.parametrize("kind,width", WIDE)
+def test_large_tets_are_as_exact_as_cell_by_cell(kind, width):
+    """Tets of 1e3 to 1e8 cells: no further off than one tet per thread, which clips each cell on its own."""
+    tets = wide(kind, width)
+    want = oracle(tets, unit_box(32), 32)
+    got, _ = blocks(tets, unit_box(32), 32)
+    assert rms(got, want) <= rms(one_per_thread(tets, unit_box(32), 32), want)
+
+
+def test_cells_inside_a_large_tet_are_full():
+    """Their mass is cell volume / tet volume, to the rounding of that quotient, whatever block they are in."""
+    t = np.array([[[-20, -21, -19], [70, -18, -15], [-17, 66, -22], [-14, -16, 75]]], np.float32)
+    v = t[0].astype(np.float64)
+    full = 6.0 / abs(np.linalg.det(v[1:] - v[0]))
+    got, _ = blocks(t, unit_box(32), 32)
+    # barycentric coordinates of the cells' corners
+    g = np.stack(np.meshgrid(*[np.arange(33.0)] * 3, indexing="ij"), -1).transpose(2, 1, 0, 3).reshape(-1, 3)
+    l = np.linalg.solve((v[1:] - v[0]).T, (g - v[0]).T).T
+    corner = (np.column_stack([l, 1.0 - l.sum(1)]) > 1e-9).all(1).reshape(33, 33, 33)
+    inner = np.all([corner[i:32 + i, j:32 + j, k:32 + k] for i in (0, 1) for j in (0, 1) for k in (0, 1)], axis=0).reshape(-1)
+    assert inner.sum() > 1000 and (got > 0).sum() > inner.sum()
+    assert np.abs(got[inner] - full).max() <= 4 * np.finfo(float).eps * full
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("mode", [A.MODE_PLAIN, A.MODE_BATCHED])
+@pytest.mark.parametrize("kind,width", WIDE)
+def test_large_tets_on_the_gpu(mode, kind, width):
+    tets = wide(kind, width)
+    want = oracle(tets, unit_box(32), 32)
+    print(f"[block deposit] {kind} {width} mode {mode}", flush=True)
+    got = A.deposit_soup(tets, unit_box(32), 32, 1.0, mode=mode)
+    cells, _ = A.deposit_soup(tets, unit_box(32), 32, 1.0, stats=True)  # one tet per thread
+    assert rms(got, want) <= rms(cells, want)
