@@ -64,6 +64,7 @@ GridDesc make_grid_desc(const GridGeom& g, long long base) {
         // it moves cell faces by at most an ulp of the index
         d.r[a] = g.scale[a] == 1.0 / g.delta[a] ? 1.0 : g.delta[a] * g.scale[a];
         d.scale[a] = g.scale[a];
+        d.scale_lo[a] = double((long double)(g.dims) / ((long double)(g.gmax[a]) - (long double)(g.gmin[a])) - (long double)(g.scale[a]));
     }
     d.cell_vol = g.cell_vol;
     d.base = base;

@@ -31,6 +31,7 @@ struct GridDesc {
     double delta[3];
     double r[3];  // delta_a * scale_a: the cell edge in the scaled coordinates (1 exactly when scale_a = 1/delta_a)
     double scale[3];
+    double scale_lo[3];  // cells per unit length = scale + scale_lo to twice the precision (block form)
     double cell_vol;
     long long base;
     int dims;

@@ -67,21 +67,26 @@ ADECO_HD void covered(double mn, double mx, int dims, int& l, int& h) {
     h = int(fmax(fmin(floor(mx + 1e-9), top), 0.0));
 }
 
-// A tet in the cells of a grid: its cover and its vertices, in the cover's axis order.
+// A tet in the cells of a grid: its cover and its vertices, from the cover's corner and in its axis order.
 struct TetCover {
     int lo[3], e[3], code;
     double s[4][3];
 };
 
+// The vertices are scaled from the corner, rounded once at their distance from it: a coordinate of 50 cells from the
+// grid's face would be off by up to 7e-15 cells, and by the scale's rounding as much again.  Grids against extended
+// precision, rms (from the face; from the corner; one tet per thread): 32^3 lattice on 64^3 cells 2.2e-15, 3.8e-16,
+// 2.4e-16; 12^3 on 28^3 2.2e-15, 3.6e-16, 1.0e-15; 24^3 on 60^3 1.9e-15, 3.6e-16, 6e-15.
 ADECO_HD TetCover cover_of(const V3<double> v[4], const GridDesc& g) {
     double c[4][3];
     int lo[3], e[3];
     for (int a = 0; a < 3; ++a) {
-        for (int q = 0; q < 4; ++q) c[q][a] = g.scale[a] * (comp(v[q], a) - g.gmin[a]);
+        for (int q = 0; q < 4; ++q) c[q][a] = comp(v[q], a) - g.gmin[a];
         int h;
-        covered(fmin(fmin(c[0][a], c[1][a]), fmin(c[2][a], c[3][a])), fmax(fmax(c[0][a], c[1][a]), fmax(c[2][a], c[3][a])), g.dims,
-                lo[a], h);
+        covered(g.scale[a] * fmin(fmin(c[0][a], c[1][a]), fmin(c[2][a], c[3][a])),
+                g.scale[a] * fmax(fmax(c[0][a], c[1][a]), fmax(c[2][a], c[3][a])), g.dims, lo[a], h);
         e[a] = h - lo[a] + 1;
+        for (int q = 0; q < 4; ++q) c[q][a] = fma(c[q][a], g.scale_lo[a], fma(c[q][a], g.scale[a], -double(lo[a])));
     }
     TetCover t;
     t.code = role_code(e);
@@ -114,7 +119,7 @@ struct Block {
     double full, scale;
 };
 
-// lo, e: the cover's first cell and extents in its axis order; s: the vertices in cells, in that order.
+// lo, e: the cover's first cell and extents in its axis order; s: the vertices from its corner, in that order.
 ADECO_HD Block make_block(const int lo[3], const int e[3], const double s[4][3], double full, unsigned unit) {
     Block b;
     b.full = full;
@@ -132,9 +137,9 @@ ADECO_HD Block make_block(const int lo[3], const int e[3], const double s[4][3],
         b.c[a] = imin(sh.b[a], e[a] - i[a] * sh.b[a]);
     }
     for (int q = 0; q < 4; ++q) {
-        b.x[q] = s[q][0] - double(b.lo[0]);
-        b.y[q] = s[q][1] - double(b.lo[1]);
-        b.z[q] = s[q][2] - double(b.lo[2]);
+        b.x[q] = s[q][0] - double(b.lo[0] - lo[0]);
+        b.y[q] = s[q][1] - double(b.lo[1] - lo[1]);
+        b.z[q] = s[q][2] - double(b.lo[2] - lo[2]);
     }
     return b;
 }

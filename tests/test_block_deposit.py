@@ -119,3 +119,66 @@ def test_large_tets_on_the_gpu(mode, kind, width):
     got = A.deposit_soup(tets, unit_box(32), 32, 1.0, mode=mode)
     cells, _ = A.deposit_soup(tets, unit_box(32), 32, 1.0, stats=True)  # one tet per thread
     assert rms(got, want) <= rms(cells, want)
+
+
+def kuhn_lattice(n, noise, scale, offset, seed):
+    """The Kuhn tets of n^3 displaced cubes."""
+    rng = np.random.default_rng(seed)
+    v = np.stack(np.meshgrid(*[np.arange(n + 1.0)] * 3, indexing="ij"), -1)
+    v = (v + rng.normal(0, noise, v.shape)) * scale + offset
+    out = []
+    for p in KUHN:
+        o, vs = np.zeros(3, int), []
+        for s in range(4):
+            vs.append(v[o[0]:o[0] + n, o[1]:o[1] + n, o[2]:o[2] + n].reshape(-1, 3))
+            if s < 3:
+                o[p[s]] += 1
+        out.append(np.stack(vs, 1))
+    return np.concatenate(out).astype(np.float32)
+
+
+def cells_in_extended_precision(tets, box, dims):
+    """Every cell of every tet on its own, its faces and coordinates in extended precision (the oracle's faces are
+    doubles): the grid."""
+    clip = O.load().oracle_clip_unit_cube_ld
+    box = box.astype(np.longdouble)
+    c = (tets.astype(np.longdouble) - box[0::2]) * dims / (box[1::2] - box[0::2])
+    grid = np.zeros((dims, dims, dims), np.longdouble)
+    for t in c:
+        a, b, d = (t[i] - t[3] for i in range(3))
+        vol = a @ np.array([b[1] * d[2] - b[2] * d[1], b[2] * d[0] - b[0] * d[2], b[0] * d[1] - b[1] * d[0]]) / 6
+        if vol < 0:  # the clip takes positively oriented tets
+            t, vol = t[[3, 1, 2, 0]], -vol
+        lo, hi = np.maximum(np.floor(t.min(0)), 0).astype(int), np.minimum(np.floor(t.max(0)), dims - 1).astype(int)
+        for i in range(lo[0], hi[0] + 1):
+            for j in range(lo[1], hi[1] + 1):
+                for k in range(lo[2], hi[2] + 1):
+                    local = np.ascontiguousarray((t - np.array([i, j, k])).astype(np.float64))
+                    grid[k, j, i] += np.longdouble(clip(A.ptr(local))) / vol
+    return grid.reshape(-1)
+
+
+def rounded_box():
+    """Tets of about a cell, 50 cells from the grid's corner, in a box whose cells are no binary fractions."""
+    tets = kuhn_lattice(5, 0.25, 2 * 0.37, 31.3 + 47 * 0.37, 12)
+    return tets, np.array([31.3, 31.3 + 60 * 0.37] * 3, np.float32), 60
+
+
+# A vertex is rounded at up to 8 cells from its cover's corner (4.4e-16, and as much in its block), which moves faces whose
+# area is about 6 times the tet's volume: 5e-15 at worst, and less than half of it rms.  Rounded at 50 cells: 7e-15.
+NEAR = 2e-15
+
+
+def test_cell_coordinates_are_rounded_near_the_tet():
+    tets, box, dims = rounded_box()
+    got, _ = blocks(tets, box, dims)
+    assert rms(got, cells_in_extended_precision(tets, box, dims)) <= NEAR
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("mode", [A.MODE_PLAIN, A.MODE_BATCHED])
+def test_cell_coordinates_on_the_gpu(mode):
+    tets, box, dims = rounded_box()
+    want = cells_in_extended_precision(tets, box, dims)
+    print(f"[block deposit] rounded box, mode {mode}", flush=True)
+    assert rms(A.deposit_soup(tets, box, dims, 1.0, mode=mode), want) <= NEAR
