@@ -12,10 +12,10 @@
 //     in the same way;
 //   * z: the share of a piece below a plane is closed form in its 4 sorted heights.
 // Only the coordinates still needed are carried: (y, z) after the x cut, z after the y cut.  A piece's
-// volume is its parent's times a product of edge ratios, so no determinant is taken and a thin tet
-// loses nothing: every share has an absolute error of a few ulps of the whole tet.  A cell whose share
-// is small against that error (kSmallShare) is recomputed alone by exact_cell_share, whose pieces do
-// not overlap and whose terms are all positive.
+// volume is its parent's times a product of edge ratios, so no determinant is taken.  A share's absolute error is a
+// few ulps of the whole tet, and of a tet (or piece of it) that is thin across y or z and cut along there, a few
+// roundings of the coordinate over the thickness.  A cell whose share is small against that error (small_share) is
+// recomputed alone by exact_cell_share, whose pieces do not overlap and whose terms are all positive.
 #pragma once
 
 #include "adeco_geom.hpp"
@@ -25,9 +25,9 @@ namespace adeco {
 // Largest number of cells in a block.
 constexpr int kBlockCells = 24;
 // Shares of a cell below kNoShare (18 ulps of the tet, which large tets are first made smaller for: the differences'
-// rounding) are empty; between that and kSmallShare they are recomputed by exact_cell_share.
+// rounding) are empty; between that and small_share() they are recomputed by exact_cell_share.
 constexpr double kNoShare = 4e-15;
-constexpr double kSmallShare = 1e-8;
+constexpr double kSmallShare = 1e-8, kThinShare = 1e-9;
 // A share this close to a whole cell's is one: a cell that lies wholly in the tet is exact.
 constexpr double kNearFull = 2e-15;
 // Tets of more than 30 cells' volume are replaced by smaller ones, block by block (shrink_tet).
@@ -148,6 +148,16 @@ struct Target {
     ADECO_HD Target(Rows xr, Rows yr, int cy, int cz_)
         : base((xr.at * cy + yr.at) * cz_), dy(yr.both ? cz_ : 0), dx(xr.both ? cy * cz_ : 0), cz(cz_) {}
 };
+
+// Shares of a tet below this are recomputed: the rounding of a cut point counts against the extents of what it
+// is cut from, so by far less in a flat tet across y or z (1e-4 cells thick and cut along, shares of 1e-8..1e-6: 1.5e-5
+// off at most with kSmallShare alone, 4e-9 so, 5e-7 one tet per thread; 3 % more recomputes of ordinary tets).  Not
+// across x, whose coordinates are the vertices' own.
+ADECO_HD double small_share(const double y[4], const double z[4]) {
+    const double ey = fmax(fmax(y[0], y[1]), fmax(y[2], y[3])) - fmin(fmin(y[0], y[1]), fmin(y[2], y[3]));
+    const double ez = fmax(fmax(z[0], z[1]), fmax(z[2], z[3])) - fmin(fmin(z[0], z[1]), fmin(z[2], z[3]));
+    return fma(kThinShare, recip(fmin(ey, ez)), kSmallShare);
+}
 
 // Adds the shares of a piece with heights z0..z3 (any order) and signed share w between the z planes
 // 0..cz, cell by cell, where t says.  Without branches but for the loop over the planes that cut it: an add

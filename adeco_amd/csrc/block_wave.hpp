@@ -135,9 +135,10 @@ __device__ __forceinline__ unsigned clip_blocks(const Loader& ld, bool on, int2 
     unsigned redo = 0u;
     if (!on) return redo;
     if (huge) return (1u << (b.c[0] * b.c[1] * b.c[2])) - 1u;
+    const double small = small_share(b.y, b.z);
     for_cells(b.c, ld.place(e, b.lo), [&](int i, int64_t at) {
         const double f = LaneShares::value(sum[i * kWaveTile]);
-        if (f >= kSmallShare) ld.add(e, at, (fabs(f - b.full) <= kNearFull ? b.full : f) * b.scale);
+        if (f >= small) ld.add(e, at, (fabs(f - b.full) <= kNearFull ? b.full : f) * b.scale);
         else if (fabs(f) >= kNoShare) redo |= 1u << i;
     });
     return redo;

@@ -331,9 +331,10 @@ extern "C" int adeco_selftest_deposit_blocks_f64(const float* tets, int64_t n_te
             LeafSums<HostShares> leaves{shares};
             const bool huge = b.full < kHugeTet;
             block_shares(!huge, b.x, b.y, b.z, b.c[0], b.c[1], b.c[2], leaves);
+            const double small = small_share(b.y, b.z);
             for_cells(b.c, p, [&](int c, int64_t at) {
                 double f = fabs(sum[c] - b.full) <= kNearFull ? b.full : sum[c], keep[15];
-                if (f < kSmallShare || huge) {
+                if (f < small || huge) {
                     if (fabs(f) < kNoShare && !huge) return;
                     const Block cell = cell_of(b, c);
                     f = exact_cell_share(cell.x, cell.y, cell.z, [&](int j) -> double& { return keep[j]; });

@@ -1,11 +1,14 @@
 """The block form of the FP64 deposit on the host: whole soups, from the covers of their tets to the cells' sums,
 against the extended-precision oracle and the one-tet-per-thread form."""
 
+from fractions import Fraction as F
+
 import numpy as np
 import pytest
 
 import adeco_amd as A
 from tests import _oracle as O
+from tests.rational_clip import tet_box_volume
 from tests.test_block_clip import soup_of_extents
 
 KUHN = [(0, 1, 2), (0, 2, 1), (1, 0, 2), (1, 2, 0), (2, 0, 1), (2, 1, 0)]
@@ -182,3 +185,49 @@ def test_cell_coordinates_on_the_gpu(mode):
     want = cells_in_extended_precision(tets, box, dims)
     print(f"[block deposit] rounded box, mode {mode}", flush=True)
     assert rms(A.deposit_soup(tets, box, dims, 1.0, mode=mode), want) <= NEAR
+
+
+# Flat tets with a share of 1e-8 to 1e-7 that the differences get wrong by 3e-6 to 1.5e-5 of itself (7 of 40 000 drawn as
+# below).
+FLAT = [
+    [[5.124186038970947, 2.7174665927886963, 2.9999868869781494], [7.428884983062744, 3.4607295989990234, 3.00002121925354],
+     [4.628147602081299, 2.9347012042999268, 3.000011444091797], [4.359897136688232, 3.0584897994995117, 3.0000274181365967]],
+    [[3.814727544784546, 5.635190963745117, 5.000024795532227], [3.1704132556915283, 5.788705348968506, 5.0000081062316895],
+     [4.357591152191162, 4.377269744873047, 4.999981880187988], [3.50095272064209, 4.846557140350342, 4.999975204467773]],
+    [[4.999984264373779, 5.610897541046143, 4.5403618812561035], [5.000033378601074, 7.301886081695557, 3.4920175075531006],
+     [5.000016689300537, 4.822857856750488, 3.4201204776763916], [5.000036239624023, 4.0167341232299805, 3.6561317443847656]],
+    [[1.9999812841415405, 7.243916034698486, 2.5601866245269775], [2.0001235008239746, 4.069445610046387, 3.419501543045044],
+     [2.0000534057617188, 3.630175828933716, 2.6255669593811035], [1.9998281002044678, 6.657833576202393, 3.228499174118042]],
+]
+
+
+def flat_tets(n):
+    rng = np.random.default_rng(2)
+    out = [np.array(FLAT)]
+    for i in range(n):
+        t = rng.uniform(2, 4, 3) + rng.uniform(0, 1, (4, 3)) * np.array([1.5, 2.5, 4.0])[rng.permutation(3)]
+        t[:, rng.integers(3)] = rng.integers(2, 6) + rng.uniform(-0.5, 0.5, 4) * [1e-3, 1e-4][i % 2]
+        out.append(t[None])
+    return np.concatenate(out).astype(np.float32)
+
+
+def volume(v):
+    a, b, c = ([v[i][k] - v[3][k] for k in range(3)] for i in range(3))
+    return abs(a[0] * (b[1] * c[2] - b[2] * c[1]) + b[0] * (c[1] * a[2] - c[2] * a[1]) + c[0] * (a[1] * b[2] - a[2] * b[1])) / 6
+
+
+def test_flat_tets_cut_along():
+    """Tets that are thin along an axis and lie across a cell face there.  A cut point is rounded to about 1e-15 cells,
+    1e-15 / thickness of a share; shares below 1e-9 / thickness are recomputed, to 1e-15 of the tet: so to that or 1e-6
+    of the share.  Small shares against rationals."""
+    checked = 0
+    for t in flat_tets(1000):
+        got, _ = blocks(t[None], unit_box(8), 8)
+        v = [tuple(F(float(x)) for x in p) for p in t]
+        for c in np.nonzero((got >= 1e-12) & (got < 1e-6))[0]:
+            lo = (int(c) % 8, int(c) // 8 % 8, int(c) // 64)
+            want = float(tet_box_volume(v, lo, tuple(i + 1 for i in lo)) / volume(v))
+            assert abs(got[c] - want) <= max(1e-15, 1e-6 * want)
+            checked += 1
+        assert abs(got.sum() - 1.0) <= 1e-9
+    assert checked > 80
