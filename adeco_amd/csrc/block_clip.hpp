@@ -159,6 +159,16 @@ ADECO_HD double small_share(const double y[4], const double z[4]) {
     return fma(kThinShare, recip(fmin(ey, ez)), kSmallShare);
 }
 
+// A share as an integer of 2^-62, and a sum of such.  Pieces reach a block's sums in an order that depends on what
+// else the wave clips, and a sum of integers does not depend on its order (the unit is far below the rounding of a
+// share, and what wraps on the way wraps back).  The lower part of a tiny negative share rounds up to 2^32, which has
+// no conversion to unsigned.
+ADECO_HD long long fixed_share(double share) {
+    const double t = share * 0x1p30, hi = floor(t);
+    return (long long)((unsigned long long)(unsigned)int(hi) << 32 | unsigned(fmin((t - hi) * 0x1p32, 4294967295.0)));
+}
+ADECO_HD double from_fixed(unsigned long long v) { return double((long long)v) * 0x1p-62; }
+
 // Adds the shares of a piece with heights z0..z3 (any order) and signed share w between the z planes
 // 0..cz, cell by cell, where t says.  Without branches but for the loop over the planes that cut it: an add
 // that does not apply adds 0 to the same cell.  Acc: term(share) a value to sum (with its negative), add(cell,

@@ -60,16 +60,10 @@ __device__ __forceinline__ void push_blocks(BlockLds& L, int lane, int key, int2
     wave_sync();
 }
 
-// A lane's column of shares, summed as integers of 2^-62: leaves reach it in an order that depends on what else
-// the wave clips, and a sum of integers does not depend on its order (the unit is far below the rounding of a
-// share, and what wraps on the way wraps back).
+// A lane's column of shares.
 struct LaneShares {
     unsigned long long* a;
-    __device__ __forceinline__ static long long term(double share) {
-        const double t = share * 0x1p30, hi = floor(t);
-        return (long long)((unsigned long long)(unsigned)int(hi) << 32 | unsigned((t - hi) * 0x1p32));
-    }
-    __device__ __forceinline__ static double value(unsigned long long v) { return double((long long)v) * 0x1p-62; }
+    __device__ __forceinline__ static long long term(double share) { return fixed_share(share); }
     __device__ __forceinline__ void add(int i, long long v) {
         __hip_atomic_fetch_add(a + i * kWaveTile, (unsigned long long)v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
     }
@@ -137,7 +131,7 @@ __device__ __forceinline__ unsigned clip_blocks(const Loader& ld, bool on, int2 
     if (huge) return (1u << (b.c[0] * b.c[1] * b.c[2])) - 1u;
     const double small = small_share(b.y, b.z);
     for_cells(b.c, ld.place(e, b.lo), [&](int i, int64_t at) {
-        const double f = LaneShares::value(sum[i * kWaveTile]);
+        const double f = from_fixed(sum[i * kWaveTile]);
         if (f >= small) ld.add(e, at, (fabs(f - b.full) <= kNearFull ? b.full : f) * b.scale);
         else if (fabs(f) >= kNoShare) redo |= 1u << i;
     });

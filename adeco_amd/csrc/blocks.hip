@@ -227,9 +227,9 @@ __global__ void __launch_bounds__(kThreads, 2) k_step_blocks(const TileSource* _
 
 // Shares summed on the host as the lanes of a wave do (the same code; tests only).
 struct HostShares {
-    double* a;
-    static double term(double share) { return share; }
-    void add(int i, double v) { a[i] += v; }
+    unsigned long long* a;
+    static long long term(double share) { return fixed_share(share); }
+    void add(int i, long long v) { a[i] += (unsigned long long)v; }
 };
 
 }  // namespace
@@ -282,11 +282,12 @@ extern "C" int adeco_selftest_block_f64(const double* t, const int* cells3, doub
         y[q] = t[3 * q + 1];
         z[q] = t[3 * q + 2];
     }
-    for (int i = 0; i < n; ++i) shares[i] = 0.0;
-    HostShares sum{shares};
-    LeafSums<HostShares> leaves{sum};
+    unsigned long long sum[kBlockCells] = {};
+    HostShares sums{sum};
+    LeafSums<HostShares> leaves{sums};
     block_shares(true, x, y, z, cx, cy, cz, leaves);
     for (int i = 0; i < n; ++i) {
+        shares[i] = from_fixed(sum[i]);
         const int k = i % cz, b = (i / cz) % cy, a = i / (cz * cy);
         double lx[4], ly[4], lz[4], keep[15];
         for (int q = 0; q < 4; ++q) {
@@ -326,14 +327,15 @@ extern "C" int adeco_selftest_deposit_blocks_f64(const float* tets, int64_t n_te
                 continue;
             }
             shrink_tet(b);
-            double sum[kBlockCells] = {};
+            unsigned long long sum[kBlockCells] = {};
             HostShares shares{sum};
             LeafSums<HostShares> leaves{shares};
             const bool huge = b.full < kHugeTet;
             block_shares(!huge, b.x, b.y, b.z, b.c[0], b.c[1], b.c[2], leaves);
             const double small = small_share(b.y, b.z);
             for_cells(b.c, p, [&](int c, int64_t at) {
-                double f = fabs(sum[c] - b.full) <= kNearFull ? b.full : sum[c], keep[15];
+                double f = from_fixed(sum[c]), keep[15];
+                if (fabs(f - b.full) <= kNearFull) f = b.full;
                 if (f < small || huge) {
                     if (fabs(f) < kNoShare && !huge) return;
                     const Block cell = cell_of(b, c);

@@ -231,3 +231,15 @@ def test_flat_tets_cut_along():
             checked += 1
         assert abs(got.sum() - 1.0) <= 1e-9
     assert checked > 80
+
+
+@pytest.mark.parametrize("depth", [1e-7, 1e-9, 1e-12])
+def test_a_vertex_just_beyond_a_face(depth):
+    """What is cut off is a share of 1e-19 to 1e-36, a negative term far below the unit of the sums."""
+    rng = np.random.default_rng(6)
+    for i in range(300):
+        t = rng.uniform(0.2, 2.0, (4, 3))
+        t[i % 4, (i // 4) % 3] = -depth
+        t = t[None].astype(np.float32)
+        got, _ = blocks(t, unit_box(8), 8)
+        assert np.abs(got - oracle(t, unit_box(8), 8)).max() <= 2e-14
