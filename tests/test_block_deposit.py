@@ -243,3 +243,25 @@ def test_a_vertex_just_beyond_a_face(depth):
         t = t[None].astype(np.float32)
         got, _ = blocks(t, unit_box(8), 8)
         assert np.abs(got - oracle(t, unit_box(8), 8)).max() <= 2e-14
+
+
+@pytest.mark.parametrize("cells", [(2, 2, 6), (1, 4, 6), (2, 3, 4), (1, 1, 24), (2, 2, 5)])
+def test_blocks_of_up_to_24_cells_match_the_rational_clip(cells):
+    """The clip of one block against rationals: 2e-14 of the tet, and where it is thin along an axis a few roundings of
+    its coordinates there (up to 24 cells: 1e-14 with those of the cut points) over the thickness."""
+    rng = np.random.default_rng(cells[2])
+    for i in range(6):
+        thickness = [0.0, 0.0, 0.0, 1e-1, 1e-2, 1e-3][i]
+        t = rng.uniform(0.2, 0.8, 3) * np.array(cells) + rng.standard_normal((4, 3)) * [0.4, 1.0, 3.0][i % 3]
+        if thickness:
+            axis = int(np.argmax(np.array(cells) > 1)) if i % 2 else 2
+            t[:, axis] = rng.integers(1, max(cells[axis], 2)) + rng.uniform(-0.5, 0.5, 4) * thickness
+        t = np.ascontiguousarray(t)
+        shares, alone, c = np.zeros(24), np.zeros(24), np.array(cells, np.int32)
+        assert A.load().adeco_selftest_block_f64(A.ptr(t), A.ptr(c), A.ptr(shares), A.ptr(alone)) == int(np.prod(cells))
+        v = [tuple(F(float(x)) for x in p) for p in t]
+        tol = 2e-14 + (1e-14 / thickness if thickness else 0.0)
+        for n, (a, b, k) in enumerate(np.ndindex(*cells)):
+            want = float(tet_box_volume(v, (a, b, k), (a + 1, b + 1, k + 1)) / volume(v))
+            assert abs(shares[n] - want) <= tol
+            assert abs(alone[n] - want) <= max(1e-15, 1e-6 * want)
