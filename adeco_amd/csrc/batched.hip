@@ -1062,7 +1062,7 @@ adeco_status deposit_leaves_direct(adeco_octree_s* T, int dims, int decompositio
     if (e == hipSuccess) e = launch_zero_u32(reinterpret_cast<unsigned*>(ctr), int(sizeof(DirectCounters) / 4), ds.stream);
     if (e == hipSuccess) e = hipEventRecord(ds.evk0, ds.stream);
     if (e == hipSuccess)
-        e = launch_direct_leaves(lv, decomposition, T->d_pairs.as<int32_t>(), pair_grid, P, T->d_leaf_geom.as<GridDesc>(), dims, small, tet_mass,
+        e = launch_direct_leaves(lv, decomposition, T->d_pairs.as<int32_t>(), pair_grid, P, T->d_leaf_geom.as<GridDesc>(), small, tet_mass,
                                  T->d_grids.as<double>(), ctr, L->device, ds.stream);
     if (e == hipSuccess) e = hipEventRecord(ds.evk1, ds.stream);
     if (e != hipSuccess) return hip_fail(e, "leaf deposit launch");

@@ -149,7 +149,7 @@ hipError_t launch_pair_grid(hipStream_t stream, const int64_t* grid_off, int n_g
 // The direct form over the (leaf, tet) pairs of an octree (direct.hip).
 bool direct_deposit_fits(const GridDesc* grids, int64_t n, int64_t n_tets);
 hipError_t launch_direct_leaves(const LatticeView& lat, int decomp, const int32_t* d_pairs, const int32_t* d_pair_grid,
-                                int64_t n_pairs, const GridDesc* d_grids, int dims, bool small_tets, double tet_mass,
+                                int64_t n_pairs, const GridDesc* d_grids, bool small_tets, double tet_mass,
                                 double* d_grid_buf, DirectCounters* ctr, int device, hipStream_t stream);
 // Leaf deposit in that form, all leaves in one launch; taken = false (and nothing done) where it does not fit, or
 // where pair lines are faster and wanted (`only_small`).

@@ -15,6 +15,8 @@ namespace adeco {
 struct BlockShape {
     int b[3], n[3];
 };
+// Blocks of the largest cover, 1023^3 cells in blocks of 2 x 2 x 6.
+constexpr unsigned kMostBlocks = 512u * 512u * 171u;
 
 ADECO_HD BlockShape block_shape(int ex, int ey, int ez) {
     static_assert(kBlockCells == 24, "block sizes");

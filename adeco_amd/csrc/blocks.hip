@@ -45,12 +45,12 @@ namespace {
 constexpr int kWaves = 4;  // wavefronts of a workgroup
 constexpr int kThreads = 64 * kWaves;
 
-// 3 workgroups of 4 waves share the 160 KB of a CU, which are handed out in pieces of 1280 bytes
+// 2 workgroups of 4 waves share the 160 KB of a CU, which are handed out in pieces of 1280 bytes
 static_assert((sizeof(BlockLds) * kWaves + 1279) / 1280 * 1280 * 2 <= 160 * 1024, "2 workgroups per CU");
 
-// A queue entry: the pair, and the block's index in it with the source slot in the upper 6 bits (a
-// pair has at most 512 * 512 * 256 = 2^26 blocks).
+// A queue entry: the pair, and the block's index in it with the source slot in the upper 6 bits.
 constexpr int kUnitBits = 26;
+static_assert(kMostBlocks <= 1u << kUnitBits, "bits of a block's index");
 constexpr unsigned kUnitMask = (1u << kUnitBits) - 1u;
 
 __global__ void __launch_bounds__(256) k_block_setup(LatticeView lat, PackedCorners ct, const int32_t* __restrict__ pairs,

@@ -235,7 +235,7 @@ __global__ void __launch_bounds__(kThreads, 2) k_deposit_direct(Tets tets, unsig
 }
 
 template <class Tets>
-hipError_t launch(const Tets& tets, int64_t n_tets, int dims, bool small_tets, double tet_mass, double* grid, DirectCounters* ctr,
+hipError_t launch(const Tets& tets, int64_t n_tets, bool small_tets, double tet_mass, double* grid, DirectCounters* ctr,
                   int device, hipStream_t stream) {
     if (n_tets <= 0) return hipSuccess;
     int cus = 256;
@@ -246,8 +246,8 @@ hipError_t launch(const Tets& tets, int64_t n_tets, int dims, bool small_tets, d
     // items per resident wave 160 us, one for half 120, for a quarter or an eighth 90-100; 98 784 tets: 343, 285,
     // 282 us; 196 608 tets on 64^3 cells: 457, 445, 440.)
     const int64_t waves = int64_t(cus) * 2 * kWaves;
-    // (64 tets of up to 2^26 blocks each would overflow their 32-bit sum on grids beyond 512^3)
-    int per_item = dims <= 512 ? 64 : 32;
+    static_assert(64ull * kMostBlocks + kWaveTile < 1ull << 32, "the blocks of an item's tets are counted in 32 bits");
+    int per_item = kWaveTile;
     while (per_item > 1 && 8 * n_tets < waves * per_item) per_item >>= 1;
     const int64_t items = (n_tets + per_item - 1) / per_item;
     const WaveLaunch w = wave_launch(items, block_occupancy(), kWaves, device);
@@ -275,25 +275,25 @@ bool direct_deposit_fits(const GridGeom& g, int64_t n_tets) {
 
 hipError_t launch_direct_lattice(const LatticeView& lat, int decomp, const int32_t* d_ids, int64_t n_tets, const GridGeom& g,
                                  double tet_mass, double* d_grid, DirectCounters* ctr, int device, hipStream_t stream) {
-    return launch(LatticeTets{{make_grid_desc(g, 0)}, lat, pack_corners(corner_table(decomp)), d_ids}, n_tets, g.dims, false, tet_mass,
+    return launch(LatticeTets{{make_grid_desc(g, 0)}, lat, pack_corners(corner_table(decomp)), d_ids}, n_tets, false, tet_mass,
                   d_grid, ctr, device, stream);
 }
 
 hipError_t launch_direct_leaves(const LatticeView& lat, int decomp, const int32_t* d_pairs, const int32_t* d_pair_grid,
-                                int64_t n_pairs, const GridDesc* d_grids, int dims, bool small_tets, double tet_mass,
+                                int64_t n_pairs, const GridDesc* d_grids, bool small_tets, double tet_mass,
                                 double* d_grid_buf, DirectCounters* ctr, int device, hipStream_t stream) {
-    return launch(LeafTets{lat, pack_corners(corner_table(decomp)), d_pairs, d_pair_grid, d_grids}, n_pairs, dims, small_tets, tet_mass,
+    return launch(LeafTets{lat, pack_corners(corner_table(decomp)), d_pairs, d_pair_grid, d_grids}, n_pairs, small_tets, tet_mass,
                   d_grid_buf, ctr, device, stream);
 }
 
 hipError_t launch_direct_soup(const float* d_tets, int64_t n_tets, const GridGeom& g, double tet_mass, double* d_grid,
                               DirectCounters* ctr, int device, hipStream_t stream) {
-    return launch(SoupTets{{make_grid_desc(g, 0)}, d_tets}, n_tets, g.dims, false, tet_mass, d_grid, ctr, device, stream);
+    return launch(SoupTets{{make_grid_desc(g, 0)}, d_tets}, n_tets, false, tet_mass, d_grid, ctr, device, stream);
 }
 
 hipError_t launch_direct_patches(const float* d_pos, int64_t num_patches, int m, int decomp, const GridGeom& g, double tet_mass,
                                  double* d_grid, DirectCounters* ctr, int device, hipStream_t stream) {
-    return launch(PatchTets{{make_grid_desc(g, 0)}, d_pos, m, pack_corners(corner_table(decomp))}, num_patches * m * m * m * 6, g.dims,
+    return launch(PatchTets{{make_grid_desc(g, 0)}, d_pos, m, pack_corners(corner_table(decomp))}, num_patches * m * m * m * 6,
                   false, tet_mass, d_grid, ctr, device, stream);
 }
 

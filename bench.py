@@ -11,7 +11,8 @@ FP64 leaf grids in HBM (the octree is built once, outside the timed region, and 
 tets/s = 6 N^3 / step time; each tet counts once however many leaves it touches.
 `--workload c2` runs the same measurement on the 128^3 lattice (rms 3 spacings, no infall).
 
-Extra fields: the plain one-tet-per-thread per-leaf-launch form measured the same way, the
+Extra fields: the plain form (all leaves straight from their (leaf, tet) pairs, as the batched one where tets are
+small) measured the same way, the largest difference from the mixed-precision form, whose clip is another, the
 hipGraph replay, the whole one-rank workflow, the total-mass drift, the roofline of the dominant
 kernel (HIP events on its launch stream; algorithmic FLOPs and bytes from the oracle's counts in
 tests/golden/c{2,3}_flops.json) and a CPU baseline: the compiled reference CPU path (oracle/_ref,
@@ -282,7 +283,7 @@ def percentiles(lat):
 def serve_study(rates, count, seed=5, max_inflight=16):
     """Serving: the resident 256^3 lattice (the 128^3 workload's field type, rms 3 spacings) answers
     Poisson streams of ROI requests; p50/p99 latency and tets/s of the continuous-batching server
-    (real-time arrivals) against serial plain-GPU processing of the same requests (one at a time,
+    (real-time arrivals) against serial plain-form processing of the same requests (the same clip, one at a time,
     arrival order: FIFO over the measured service times)."""
     import threading
     t0 = time.perf_counter()
@@ -428,7 +429,7 @@ def heavy_tail_study(dims_list=(16, 32), n=256, steps=3):
     """The heavy-tailed batched workload: a 256^3 lattice (100,663,296 Kuhn tets) at rms 4 spacings
     with 64 seeded spherical infall centres (radius 2-8 Mpc/h), the reference octree (depth <= 6,
     split above 50,000 estimated tets) and 16^3 or 32^3-cell leaves.  The batched form (autotuned
-    launch shape; eager and hipGraph replay) against the plain per-leaf launches."""
+    launch shape; eager and hipGraph replay) against the plain form (straight from the pairs)."""
     t0 = time.perf_counter()
     log(f"[c3] generating the {n}^3 lattice with 64 infall centres")
     lat = make_lattice(n, 4.0, seed=3, infall_centres=64)
@@ -602,8 +603,8 @@ def boundary_study(reps=2):
     workload, called as the reference's worker calls it (AdDynamicLoadBalancing.h:200-205): once
     per octree leaf, with the leaf's gathered meta-patches in host memory (its meta-cell list, the
     reference's gather order), the leaf's float box, 16^3 cells, the reference's tets of mass 1,
-    into a zeroed float grid.  The plain form (straight from the patches) against the batched form; host-to-device copies of the patches and the grid
-    readback are inside the timed loop."""
+    into a zeroed float grid.  The plain form (straight from the patches) against the batched form;
+    host-to-device copies of the patches and the grid readback are inside the timed loop."""
     from adeco_amd.lattice import meta_patches
     lat = make_lattice(N, RMS, seed=SEED)
     with A.ResidentLattice.from_lattice(lat) as rl, A.Octree(rl, MAX_TETS, MAX_LEVEL) as tree:
@@ -669,7 +670,7 @@ def main():
         sys.exit(2)
     if args.heavy_tail:
         res = heavy_tail_study()
-        print(json.dumps({"metric": "tets/s exact deposit, batched vs plain per-leaf launches", "unit": "tets/s",
+        print(json.dumps({"metric": "tets/s exact deposit, batched vs plain form", "unit": "tets/s",
                           "higher_is_better": True, "n_gpus": 1, "dtype": "f64",
                           "data": "synthetic (256^3 lattice, rms 4 spacings + 64 infall centres)", **res}))
         return
@@ -798,7 +799,7 @@ def headline(args):
             log(f"[bench] batched fp64 {DIMS_FINE}^3 leaves: {wall_f / steps_f * 1e3:.2f} ms/step, kernel {main_f:.2f} ms "
                 f"({extra['fine_leaves']['tets_per_s']:.3e} tets/s)")
             A.set_launch_shape(shape["chunk"], shape["blocks_per_cu"])
-            # the plain one-tet-per-thread form, one launch per leaf
+            # the plain form: all leaves in one launch, straight from their (leaf, tet) pairs
             steps_p = 1 if n > 128 else max(2, args.steps // 2)
             wall_p, main_p, _ = run_steps(tree, steps_p, 0 if n > 128 else 1, A.MODE_PLAIN, A.PREC_FP64, decomp)
             plain_tets = lat.num_tets / (wall_p / steps_p)
@@ -806,10 +807,16 @@ def headline(args):
             tree.deposit(DIMS, decomposition=decomp, tet_mass=TET_MASS, mode=A.MODE_BATCHED, precision=A.PREC_FP64)
             extra["plain_tets_per_s"] = plain_tets
             extra["batched_over_plain"] = value / plain_tets
-            extra["plain_vs_batched_max_rel_err"] = max_rel_err(plain_grids, tree.leaf_grids(), 1e-8 * TET_MASS)
+            grids = tree.leaf_grids()
+            extra["plain_vs_batched_max_rel_err"] = max_rel_err(plain_grids, grids, 1e-8 * TET_MASS)
             del plain_grids
+            # both run the same clip at this size: the mixed-precision form's is independent of it
+            tree.deposit(DIMS, decomposition=decomp, tet_mass=TET_MASS, mode=A.MODE_BATCHED, precision=A.PREC_MIXED)
+            extra["mixed_vs_fp64_max_rel_err"] = max_rel_err(tree.leaf_grids(), grids, 1e-8 * TET_MASS)
+            del grids
             log(f"[bench] plain fp64: {wall_p / steps_p * 1e3:.2f} ms/step, {plain_tets:.3e} tets/s, "
-                f"batched/plain {extra['batched_over_plain']:.1f}x, max rel diff {extra['plain_vs_batched_max_rel_err']:.1e}")
+                f"batched/plain {extra['batched_over_plain']:.1f}x, max rel diff {extra['plain_vs_batched_max_rel_err']:.1e}, "
+                f"mixed {extra['mixed_vs_fp64_max_rel_err']:.1e}")
             # the reference's own (non-tiling) decomposition, like for like with the CPU baseline
             tree.bin(A.DECOMP_REF_EFFECTIVE)
             wall_r, _, _ = run_steps(tree, max(2, args.steps // 2), 1, A.MODE_BATCHED, A.PREC_FP64, A.DECOMP_REF_EFFECTIVE)
