@@ -19,13 +19,13 @@
 // each inner plane twice over and through up to four nested stages of full 3-D pieces.  Here a plane is
 // cut once for the cells on both its sides, a cut carries only the coordinates still needed and a
 // piece's volume comes from edge ratios (4-5x fewer instructions per tet).  256^3 clustered lattice,
-// 16^3-cell leaves, 126 M pairs: 31.4 ms against 65.6 for the column form; 128^3: 3.8 against 7.1;
-// 32^3-cell leaves on 97^3: 15.3 against 27.5, and 9.2 with the pieces gathered over the lanes and blocks of
+// 16^3-cell leaves, 126 M pairs: 31.6 ms against 65.6 for the column form; 128^3: 3.7 against 7.1;
+// 32^3-cell leaves on 97^3: 15.3 against 27.5, and 9.6 with the pieces gathered over the lanes and blocks of
 // 24 cells (block_wave.hpp).  It is also more accurate (128^3 leaf grids against 64-bit exact clipping:
-// 5e-15 against 2e-13).  What bounds it: vector instructions (issued 80 % of the time with large tets, 55 %
-// with small ones) at 65-75 % lane use, and FP64 atomics (one per cell a tet meets; the card takes 25-31 G/s
-// of them scattered).  Two workgroups of 4 waves per CU: 20 KB of LDS a
-// wave, and no spills (205 VGPRs; at 168 and 3 workgroups about 45 are spilled around each pass).
+// 5e-15 against 2e-13).  What bounds it: vector instructions (issued 80 % of the time with large tets, 52 %
+// with small ones) at 65-75 % lane use, waiting at 2 waves per SIMD, and with small tets FP64 atomics (one per cell
+// a tet meets: 17 % of the kernel, by a copy without them).  Two workgroups of 4 waves per CU: 20 KB of LDS a
+// wave, and no spills (208 VGPRs; at 168 and 3 workgroups about 45 are spilled around each pass).
 #include <hip/hip_runtime.h>
 
 #include <algorithm>

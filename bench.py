@@ -64,7 +64,7 @@ HBM_PEAK_GBS = 8000.0
 # HBM bytes per launch of the FP64 leaf deposit (k_deposit_direct) at 16^3-cell leaves: rocprofv3
 # FETCH_SIZE and WRITE_SIZE (KiB per dispatch) scaled by what each reads for a 1 GiB copy (2.0 and
 # 1.0), profiles/deposit_blocks.md (256^3 infall workload and 128^3)
-TRAFFIC_BYTES = {"c3": 5919428.9375 * 2 * 1024 + 19562973.875 * 1024, "c2": 528110.8125 * 2 * 1024 + 2061348.8125 * 1024}
+TRAFFIC_BYTES = {"c3": 5944210.390625 * 2 * 1024 + 19566232.9453125 * 1024, "c2": 530344.34375 * 2 * 1024 + 2061334.78125 * 1024}
 
 
 def log(*a):
