@@ -10,10 +10,10 @@
 #include <cmath>
 #include <cstdio>
 #include <cstring>
+#include <exception>
 #include <memory>
 #include <mutex>
 #include <string>
-#include <system_error>
 #include <thread>
 #include <vector>
 
@@ -62,24 +62,30 @@ DeviceState& device_state(int dev) {
 // From here on a download is split: a part costs a thread (about 50 us).
 constexpr size_t kSplitDownload = size_t(8) << 20;
 
+// The streams of a split download; false where they cannot be had.
+static bool download_streams(DeviceState& ds) {
+    std::lock_guard<std::mutex> lk(ds.down_mutex);
+    for (hipStream_t& s : ds.down)
+        if (!s && hipStreamCreateWithFlags(&s, hipStreamNonBlocking) != hipSuccess) {
+            s = nullptr;
+            (void)hipGetLastError();
+            return false;
+        }
+    return true;
+}
+
 // A copy to ordinary memory runs at the rate of one host thread: it moves the data out of the runtime's pinned
 // buffers, and takes a page fault for each page of a fresh array.  In four parts, each with a thread and a
 // stream of its own, 134 MB into a fresh array take 4.0 ms instead of 13.0 (16 MB 0.58 instead of 1.57); below
-// the split one copy is as fast.
+// the split one copy is as fast, and without the streams or a thread it still does.
 hipError_t download(DeviceState& ds, hipStream_t stream, void* dst, const void* src, size_t bytes) {
-    hipError_t e = hipSuccess;
-    if (bytes < kSplitDownload) {
-        e = hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, stream);
+    if (bytes < kSplitDownload || !download_streams(ds)) {
+        const hipError_t e = hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, stream);
         return e == hipSuccess ? hipStreamSynchronize(stream) : e;
     }
     constexpr int kParts = DeviceState::kDownloads;
     const int dev = ds.id;
-    e = hipStreamSynchronize(stream);
-    {
-        std::lock_guard<std::mutex> lk(ds.down_mutex);
-        for (int i = 0; i < kParts && e == hipSuccess; ++i)
-            if (!ds.down[i]) e = hipStreamCreateWithFlags(&ds.down[i], hipStreamNonBlocking);
-    }
+    const hipError_t e = hipStreamSynchronize(stream);
     if (e != hipSuccess) return e;
     const size_t part = bytes / kParts & ~size_t(4095);
     hipError_t result[kParts];
@@ -95,7 +101,7 @@ hipError_t download(DeviceState& ds, hipStream_t stream, void* dst, const void* 
     for (int i = 1; i < kParts; ++i) {
         try {
             threads[i] = std::thread(copy, i);
-        } catch (const std::system_error&) {
+        } catch (const std::exception&) {
             copy(i);  // no thread to be had
         }
     }
