@@ -237,7 +237,6 @@ adeco_status deposit_patches_on_device(int dev, size_t first_patch, size_t n_pat
     if ((st = ds.grid.reserve(grid_bytes + kCountersBytes))) return st;
     if ((st = ds.pos.reserve(patches_per_pass * patch_bytes))) return st;
     DevBuf& soup = ds.soup;
-    if (batched && (st = soup.reserve(patches_per_pass * soup_bytes))) return st;
     const GridGeom g = make_grid_geom(bbox, dims, cell_scaling());
     double* d_grid = ds.grid.as<double>();
     DirectCounters* ctr = counters_after(d_grid, int64_t(ncell));
@@ -254,6 +253,7 @@ adeco_status deposit_patches_on_device(int dev, size_t first_patch, size_t n_pat
         // map or read-back: 80 patches on 24^3 cells, the call 277 -> 228 us
         counted = batched && precision == ADECO_PREC_FP64 && direct && np * tets_per_patch >= 4 * ncell;
         if (batched && !counted) {
+            if ((st = soup.reserve(patches_per_pass * soup_bytes))) return st;
             e = launch_patches_to_soup(ds.pos.as<float>(), int64_t(np), m, decomp, soup.as<float>(), ds.stream);
             if (e != hipSuccess) return hip_fail(e, "patch expansion");
             if ((st = deposit_soup_batched(ds, soup.as<float>(), int64_t(np * tets_per_patch), g, tet_mass, precision,
