@@ -894,8 +894,8 @@ static void enqueue_candidate_space(hipStream_t stream, const LatticeView& lat, 
     if (n_pairs == 0) return;
     if (pair_grid) (void)launch_pair_grid(stream, grid_off, n_grids, n_pairs, pair_grid);
     if (form == kFormBlocks)
-        (void)launch_block_setup(stream, lat, ct, pairs, n_pairs, n_dev, grid_off, n_grids, pair_grid, d_grids, tet_mass,
-                                 cs.cand, cs.pd);
+        (void)launch_block_setup(stream, lat, ct, pairs, n_pairs, n_dev, grid_off, n_grids, pair_grid, d_grids, cs.cand,
+                                 cs.pd);
     else
         hipLaunchKernelGGL(k_pair_setup, dim3(unsigned((n_pairs + 255) / 256)), dim3(256), 0, stream, lat, ct, pairs, n_pairs,
                            n_dev, grid_off, n_grids, pair_grid, d_grids, tet_mass, form == kFormFp64 ? kMaxSeg : 1, cs.cand,

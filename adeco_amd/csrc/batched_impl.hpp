@@ -158,7 +158,7 @@ adeco_status deposit_leaves_direct(adeco_octree_s* T, int dims, int decompositio
 // The block form's kernels (blocks.hip).
 hipError_t launch_block_setup(hipStream_t stream, const LatticeView& lat, const PackedCorners& ct, const int32_t* pairs,
                               int64_t n_pairs, const int64_t* n_dev, const int64_t* grid_off, int n_grids,
-                              const int32_t* pair_grid, const GridDesc* d_grids, double tet_mass, unsigned* cand, PairData* pd);
+                              const int32_t* pair_grid, const GridDesc* d_grids, unsigned* cand, PairData* pd);
 int block_occupancy();
 hipError_t launch_block_tiles(hipStream_t stream, const TileSource& src, unsigned* queue_counter,
                               unsigned long long* counters, int device);

@@ -57,8 +57,8 @@ __global__ void __launch_bounds__(256) k_block_setup(LatticeView lat, PackedCorn
                                                      int64_t n_pairs, const int64_t* __restrict__ n_dev,
                                                      const int64_t* __restrict__ grid_off, int n_grids,
                                                      const int32_t* __restrict__ pair_grid,
-                                                     const GridDesc* __restrict__ grids, double tet_mass,
-                                                     unsigned* __restrict__ cand, PairData* __restrict__ pd) {
+                                                     const GridDesc* __restrict__ grids, unsigned* __restrict__ cand,
+                                                     PairData* __restrict__ pd) {
     // lines assembled in LDS rows of an odd number of words and stored as the block's contiguous,
     // non-temporal rows
     constexpr int kWords = int(sizeof(PairData) / 8);
@@ -236,9 +236,9 @@ struct HostShares {
 
 hipError_t launch_block_setup(hipStream_t stream, const LatticeView& lat, const PackedCorners& ct, const int32_t* pairs,
                               int64_t n_pairs, const int64_t* n_dev, const int64_t* grid_off, int n_grids,
-                              const int32_t* pair_grid, const GridDesc* d_grids, double tet_mass, unsigned* cand, PairData* pd) {
+                              const int32_t* pair_grid, const GridDesc* d_grids, unsigned* cand, PairData* pd) {
     hipLaunchKernelGGL(k_block_setup, dim3(unsigned((n_pairs + 255) / 256)), dim3(256), 0, stream, lat, ct, pairs, n_pairs,
-                       n_dev, grid_off, n_grids, pair_grid, d_grids, tet_mass, cand, pd);
+                       n_dev, grid_off, n_grids, pair_grid, d_grids, cand, pd);
     return hipGetLastError();
 }
 
